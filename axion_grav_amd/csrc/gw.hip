@@ -240,6 +240,84 @@ __global__ void __launch_bounds__((TX / 2) * (N / 8)) gw_ypass_p2w_kernel(const 
     }
 }
 
+// Polarization geometry of one wavevector: z = nz/|n| and r = |n_xy|/|n| (one reciprocal; 0 at k = 0,
+// which is zeroed after the projection), rho2 = |n_xy|^2 and rho its root.
+template <typename T> __device__ __forceinline__ void z_geom(T rho2, T rho, int nz, T& z, T& r)
+{
+#pragma clang fp contract(off)
+    const T q = sqrt(rho2 + (T)nz * (T)nz);
+    const T iq = q > 0 ? (T)1 / q : (T)0;
+    z = (T)nz * iq;
+    r = rho * iq;
+}
+
+// pol_ij d into sp (pol d) and sn (conj(pol) d) for component c, (i,j) in the reference's order
+// (1,1),(2,1),(2,2),(3,1),(3,2),(3,3) (grav_waves.f90:213-247)
+template <typename T>
+__device__ __forceinline__ void z_project(int c, T ge, T re, T gc, T gs, typename V2<T>::type d, typename V2<T>::type& sp,
+                                          typename V2<T>::type& sn)
+{
+#pragma clang fp contract(off)
+    using T2 = typename V2<T>::type;
+    const int ii = c == 0 ? 0 : (c <= 2 ? 1 : 2);
+    const int jj = (c == 0 || c == 1 || c == 3) ? 0 : ((c == 2 || c == 4) ? 1 : 2);
+    const T2 p1 = {ge * gc, -gs}, p2 = {ge * gs, gc}, p3 = {-re, 0};
+    const T2 a = ii == 0 ? p1 : (ii == 1 ? p2 : p3);
+    const T2 bb = jj == 0 ? p1 : (jj == 1 ? p2 : p3);
+    T2 pol = {a.x * bb.x - a.y * bb.y, a.x * bb.y + a.y * bb.x};
+    if (ii == jj) {
+        pol.x = pol.x / 2;
+        pol.y = pol.y / 2;
+    }
+    sp.x += pol.x * d.x - pol.y * d.y;
+    sp.y += pol.x * d.y + pol.y * d.x;
+    sn.x += pol.x * d.x + pol.y * d.y;
+    sn.y += pol.x * d.y - pol.y * d.x;
+}
+
+// cos and sin of the phase q tau, in FP64 (large arguments); FP32 storage evaluates the reduced phase
+// in FP32
+template <typename T> __device__ __forceinline__ void z_phase(int64_t n2, const GwStepScalars& g, T& cq, T& sq)
+{
+#pragma clang fp contract(off)
+    double q = sqrt((double)n2) * g.dwav * g.tau;
+    if constexpr (sizeof(T) == 8) {
+        cq = cos(q);
+        sq = sin(q);
+    } else {
+        const double twopi = 6.283185307179586476925286766559;
+        float r = (float)(q - twopi * rint(q * (1.0 / twopi)));
+        __sincosf(r, &sq, &cq);
+    }
+}
+
+// The updates of grav_waves.f90:239-242 on the accumulators' old values a11, a22, a12 (and a21(),
+// which the index quirk discards) of one wavevector, written to A + m * ms; d6 is the transformed
+// (3,3) source.
+template <typename T, typename F>
+__device__ __forceinline__ void z_update(typename V2<T>::type* __restrict__ A, int64_t ms, const GwStepScalars& g, T dw, T cq,
+                                         T sq, int64_t rho2, int64_t n2, typename V2<T>::type sp, typename V2<T>::type sn,
+                                         typename V2<T>::type d6, typename V2<T>::type a11, typename V2<T>::type a22,
+                                         typename V2<T>::type a12, F&& a21_old)
+{
+#pragma clang fp contract(off)
+    using T2 = typename V2<T>::type;
+    const T2 SP = {sp.x * dw, sp.y * dw};
+    const T2 SN = {sn.x * dw, sn.y * dw};
+    st_stream(A, T2{a11.x + cq * SP.x, a11.y + cq * SP.y});
+    st_stream(A + 3 * ms, T2{a22.x + sq * SN.x, a22.y + sq * SN.y});
+    if (!g.fix_swap) {
+        T2 r12 = {a12.x + (sq * SP.x + cq * SN.x), a12.y + (sq * SP.y + cq * SN.y)};
+        const T n6 = n2 > 0 ? ((T)rho2 / (T)n2) / 2 * dw : (T)0;  // pol_33 dw = r^2/2 dw
+        st_stream(A + 2 * ms, r12);
+        st_stream(A + ms, T2{r12.x - cq * (n6 * d6.x), r12.y - cq * (n6 * d6.y)});
+    } else {
+        const T2 a21 = a21_old();
+        st_stream(A + ms, T2{a21.x + sq * SP.x, a21.y + sq * SP.y});
+        st_stream(A + 2 * ms, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
+    }
+}
+
 template <typename T, int N>
 __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel(const typename V2<T>::type* __restrict__ W,
                                                                            typename V2<T>::type* __restrict__ A,
@@ -449,6 +527,107 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
             st_stream(A + 2 * ms + ai, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
         }
         __builtin_amdgcn_sched_barrier(0);  // keep the k-points' loads from piling up in registers
+    }
+}
+
+// The same pass for the small lattices, whose grids the kernel above leaves mostly idle: a few hundred
+// short blocks, each a chain of six loads, transforms and barriers and then eight wavevectors a
+// thread, so the pass takes their latency and not their bytes.  The block takes the same tile
+// with six times the threads: thread group c transforms component c, all six at once, into its own
+// LDS tile; then the threads share the tile's wavevectors (at most two each), whose accumulators
+// were loaded before the transforms.  Same arithmetic in the same order, so the accumulators are the
+// same bit for bit.  Kernel, us: 32^3 FP64 20.7 -> 7.6, FP32C 13.6 -> 7.6; 64^3 FP64 21.6 ->
+// 13.6, FP32C 17.6 -> 9.0; 96^3 FP64 36 -> 32.  Taken where the block fits 1024 threads and its
+// six tiles 80 KiB (two blocks a CU): FP64 to N = 96, FP32 to N = 64 (128^3 FP64, 96 KiB and one
+// block a CU, was slower, 56 -> 60 us), and where the grid's waves fit the chip at once: four
+// stacked 64^3 FP32C lattices (9216 waves) step in 66 us by themselves instead of 70, but beside
+// the other stacks of a mixed batch the larger blocks cost it 1 %.
+template <typename T, int N> constexpr int p2_zpar_threads() { return 6 * p2_ztx<T, N>() * (N / 8); }
+template <typename T, int N> constexpr bool p2_zpar()
+{
+    return p2_zpar_threads<T, N>() <= 1024 && 6 * N * p2_ztx<T, N>() * (int)sizeof(typename V2<T>::type) <= 80 * 1024;
+}
+
+constexpr int64_t ZPAR_WAVES = 8192;  // 256 CUs x 4 SIMDs x 8 waves
+
+template <typename T, int N>
+__global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel(
+    const typename V2<T>::type* __restrict__ W, typename V2<T>::type* __restrict__ A,
+    const typename V2<T>::type* __restrict__ tw, GwStepScalars g, StepRef sr, const LatRef* __restrict__ lat)
+{
+#pragma clang fp contract(off)
+    if (lat) {
+        W = (const typename V2<T>::type*)lat[blockIdx.z].W2;
+        A = (typename V2<T>::type*)lat[blockIdx.z].A;
+        sr.tab = lat[blockIdx.z].tab;
+    }
+    if (const StepEntry* se = step_entry(sr)) {
+        g.tau = se->tau;
+        g.dw = se->dw;
+    }
+    using L = TiledLayout<N, p2_ztx<T, N>()>;
+    using T2 = typename V2<T>::type;
+    constexpr int TX = p2_ztx<T, N>(), TPT = N / 8, NH = N / 2 + 1, NT = p2_zpar_threads<T, N>(), TILE = N * TX;
+    constexpr int KPT = (TILE + NT - 1) / NT;
+    __shared__ T2 s[6 * TILE];
+    const int c = threadIdx.x / (TX * TPT), lt = threadIdx.x % (TX * TPT);
+    const int b = lt % TX, j0 = lt / TX;
+    const int ky = blockIdx.y, kx0 = blockIdx.x * TX;
+    const int64_t tile0 = L::idx(0, 0, ky, kx0);
+    constexpr int64_t ms = L::COMP;
+    P2Tw<T, N> twr;
+    if constexpr (sizeof(T) == 4) twr = p2_load_twiddles<T, N, +1>(j0, tw);
+    T2 v[8];
+    const bool ok = kx0 + b < NH;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = ok ? W[c * ms + tile0 + (j0 + e * TPT) * TX + b] : T2{0, 0};
+    T2 a11[KPT], a22[KPT], a12[KPT], a21[KPT];
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const int t = threadIdx.x + i * NT;
+        if (t < TILE && kx0 + t % TX < NH) {
+            a11[i] = A[tile0 + t];
+            a22[i] = A[3 * ms + tile0 + t];
+            a12[i] = A[2 * ms + tile0 + t];
+            if (g.fix_swap) a21[i] = A[ms + tile0 + t];
+        }
+    }
+    T2* sc = s + c * TILE;
+    if constexpr (sizeof(T) == 4) fft_p2<T, N, +1>(v, j0, sc, TX, b, twr);
+    else fft_p2<T, N, +1>(v, j0, sc, TX, b, P2TwTable<T, N, +1>{tw, j0});
+#pragma unroll
+    for (int e = 0; e < 8; e++) sc[(j0 + e * TPT) * TX + b] = v[e];
+    __syncthreads();
+    const int ny = wrapn(ky, N);
+    const T dw = (T)g.dw;
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const int t = threadIdx.x + i * NT;
+        if (t >= TILE) break;
+        const int kz = t / TX, kx = kx0 + t % TX;
+        if (kx >= NH) {
+            // padding columns as in the kernel above
+            if constexpr (sizeof(T) == 8)
+#pragma unroll
+                for (int m = 0; m < 4; m++) A[m * ms + tile0 + t] = T2{0, 0};
+            continue;
+        }
+        const int nx = wrapn(kx, N), nz = wrapn(kz, N);
+        const T rho2g = (T)nx * (T)nx + (T)ny * (T)ny, rhog = sqrt(rho2g);
+        T gc = 1, gs = 0, ge, re;
+        if (rhog > 0) { gc = (T)nx / rhog; gs = (T)ny / rhog; }
+        z_geom<T>(rho2g, rhog, nz, ge, re);
+        T2 sp = {0, 0}, sn = {0, 0}, d = {0, 0};
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            d = s[k * TILE + t];
+            z_project<T>(k, ge, re, gc, gs, d, sp, sn);
+        }
+        const int64_t rho2 = (int64_t)nx * nx + (int64_t)ny * ny, n2 = rho2 + (int64_t)nz * nz;
+        if (n2 == 0) sp = sn = T2{0, 0};  // k = 0: pol = 0
+        T cq, sq;
+        z_phase<T>(n2, g, cq, sq);
+        z_update<T>(A + tile0 + t, ms, g, dw, cq, sq, rho2, n2, sp, sn, d, a11[i], a22[i], a12[i], [&] { return a21[i]; });
     }
 }
 
@@ -837,6 +1016,14 @@ void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A
         constexpr int TXP = p2_ztx<T, NN>();
         if (!TiledLayout<NN, TXP>::matches(L))
             throw Error(AXG_EINVAL, "accumulation layout does not match the z pass tile");
+        if constexpr (p2_zpar<T, NN>()) {
+            constexpr int NT = p2_zpar_threads<T, NN>();
+            if ((int64_t)L.ntile * NN * nlat * (NT / 64) <= ZPAR_WAVES) {
+                hipLaunchKernelGGL((gw_zpass_par_kernel<T, NN>), dim3(L.ntile, NN, nlat), dim3(NT), 0, s, (const T2*)W,
+                                   (T2*)A, (const T2*)tw, g, sr, lat);
+                return;
+            }
+        }
         hipLaunchKernelGGL((gw_zpass_p2_kernel<T, NN>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
                            (const T2*)W, (T2*)A, (const T2*)tw, g, sr, lat);
     });
