@@ -9,11 +9,12 @@ template <typename T> struct V2;
 template <> struct V2<double> { using type = double2; };
 template <> struct V2<float> { using type = float2; };
 
-// The lattice sizes with compile-time kernels (fft_p2.h): N = 2^L in 16..1024 and
-// N = 3 * 2^L in 24..768.  Other sizes run the runtime-plan kernels.
+// The lattice sizes with compile-time kernels (fft_p2.h): N = 2^L in 16..1024, N = 3 * 2^L in
+// 24..768 and N = 3^b * 2^L, b >= 2, L >= 3, in 72..864.  Other sizes run the runtime-plan kernels.
 constexpr bool p2_size(int n)
 {
-    const int pw = n % 3 == 0 ? n / 3 : n;
+    int pw = n;
+    while (pw % 3 == 0) pw /= 3;
     return pw >= 8 && (pw & (pw - 1)) == 0 && n >= 16 && n <= 1024;
 }
 

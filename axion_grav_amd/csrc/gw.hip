@@ -38,7 +38,7 @@ template <typename T> int col_width(int N)
 // VGPRs, no pipelining), so the y pass writes 128-byte (512) or 64-byte (1024) tile rows
 // instead of half of that.  Measured: y pass 1.80 -> 1.55 ms at 512^3 and 35 -> 15 ms at
 // 1024^3, z pass within 3 %.
-template <typename T, int N> constexpr bool p2_zwide() { return sizeof(T) == 4 && N >= 512; }
+template <typename T, int N> constexpr bool p2_zwide() { return sizeof(T) == 4 && N >= 512 && !P2<N>::R9; }
 template <typename T, int N> constexpr int p2_ztx()
 {
     int tx = p2_tx<T, N>();
@@ -545,7 +545,7 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
 template <typename T, int N> constexpr int p2_zpar_threads() { return 6 * p2_ztx<T, N>() * (N / 8); }
 template <typename T, int N> constexpr bool p2_zpar()
 {
-    return p2_zpar_threads<T, N>() <= 1024 && 6 * N * p2_ztx<T, N>() * (int)sizeof(typename V2<T>::type) <= 80 * 1024;
+    return !(sizeof(T) == 4 && P2<N>::R9) && p2_zpar_threads<T, N>() <= 1024 && 6 * N * p2_ztx<T, N>() * (int)sizeof(typename V2<T>::type) <= 80 * 1024;
 }
 
 constexpr int64_t ZPAR_WAVES = 8192;  // 256 CUs x 4 SIMDs x 8 waves
@@ -628,6 +628,131 @@ __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel
         T cq, sq;
         z_phase<T>(n2, g, cq, sq);
         z_update<T>(A + tile0 + t, ms, g, dw, cq, sq, rho2, n2, sp, sn, d, a11[i], a22[i], a12[i], [&] { return a21[i]; });
+    }
+}
+
+// Polarisation vector of a mode n != 0 (grav_waves.f90:165-183): qhat = n / |n|, its azimuth
+// (cos, sin) and r = |qhat_xy|, and p1 = (qz c, -s), p2 = (qz s, c), p3 = (-r, 0).
+template <typename T> __device__ __forceinline__ void pol_hat(T& qx, T& qy, T& qz)
+{
+    T q = sqrt(qx * qx + qy * qy + qz * qz);
+    qx = qx / q; qy = qy / q; qz = qz / q;
+}
+template <typename T> __device__ __forceinline__ void pol_azimuth(T qx, T qy, T& r, T& c, T& s)
+{
+    r = sqrt(qx * qx + qy * qy);
+    if (r > 0) { c = qx / r; s = qy / r; }
+    else { c = 1; s = 0; }
+}
+template <typename T>
+__device__ __forceinline__ void pol_vec(int nx, int ny, int nz, typename V2<T>::type* p)
+{
+    T qx = (T)nx, qy = (T)ny, qz = (T)nz, r, c, s;
+    pol_hat(qx, qy, qz);
+    pol_azimuth(qx, qy, r, c, s);
+    p[0] = {qz * c, -s};
+    p[1] = {qz * s, c};
+    p[2] = {-r, 0};
+}
+
+// The z pass of the FP32 storages at N = 3^b * 2^L, b >= 2: the tile, transforms and loads ahead of
+// gw_zpass_p2_kernel with the projection and update of gw_zpass_acc_kernel (each component of qhat
+// divided by |n|, the update in FP64), which these sizes' accumulators have been made with.  The
+// polarisation vectors are formed once per wavevector.
+template <int N>
+__global__ void __launch_bounds__((p2_ztx<float, N>() * (N / 8))) gw_zpass_p9_kernel(const float2* __restrict__ W,
+                                                                              float2* __restrict__ A,
+                                                                              const float2* __restrict__ tw,
+                                                                              GwStepScalars g, StepRef sr,
+                                                                              const LatRef* __restrict__ lat)
+{
+#pragma clang fp contract(off)
+    if (lat) {
+        W = (const float2*)lat[blockIdx.z].W2;
+        A = (float2*)lat[blockIdx.z].A;
+        sr.tab = lat[blockIdx.z].tab;
+    }
+    if (const StepEntry* se = step_entry(sr)) {
+        g.tau = se->tau;
+        g.dw = se->dw;
+    }
+    using L = TiledLayout<N, p2_ztx<float, N>()>;
+    constexpr int TX = p2_ztx<float, N>(), TPT = N / 8, NH = N / 2 + 1;
+    constexpr int64_t ms = L::COMP;
+    __shared__ float2 s[N * TX];
+    const int b = threadIdx.x % TX, j0 = threadIdx.x / TX;
+    const int kx = blockIdx.x * TX + b, ky = blockIdx.y;
+    const bool ok = kx < NH;
+    const int nx = wrapn(kx, N), ny = wrapn(ky, N);
+    const int64_t tile0 = L::idx(0, 0, ky, blockIdx.x * TX) + b;
+    const P2Tw<float, N> tws = p2_load_twiddles<float, N, +1>(j0, tw);
+    float2 v[8], nxt[8], sp[8], sn[8];
+    float pz[8], pr[8], pc[8], ps[8];  // qz, r, cos and sin of the azimuth, per wavevector
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        nxt[e] = ok ? ld_stream(W + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
+        sp[e] = sn[e] = float2{0, 0};
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        float qx = (float)nx, qy = (float)ny, qz = (float)wrapn(j0 + e * TPT, N);
+        pol_hat(qx, qy, qz);
+        pz[e] = qz;
+        pol_azimuth(qx, qy, pr[e], pc[e], ps[e]);
+    }
+#pragma unroll 1
+    for (int c = 0; c < 6; c++) {
+        const int ii = c == 0 ? 0 : (c <= 2 ? 1 : 2);
+        const int jj = (c == 0 || c == 1 || c == 3) ? 0 : ((c == 2 || c == 4) ? 1 : 2);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = nxt[e];
+        if (c + 1 < 6) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                nxt[e] = ok ? ld_stream(W + (c + 1) * ms + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
+        }
+        if (c > 0) __syncthreads();
+        fft_p2<float, N, +1>(v, j0, s, TX, b, tws);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float2 p1 = {pz[e] * pc[e], -ps[e]}, p2 = {pz[e] * ps[e], pc[e]}, p3 = {-pr[e], 0};
+            const float2 a = ii == 0 ? p1 : (ii == 1 ? p2 : p3), bb = jj == 0 ? p1 : (jj == 1 ? p2 : p3);
+            float2 pol = {a.x * bb.x - a.y * bb.y, a.x * bb.y + a.y * bb.x};
+            if (ii == jj) { pol.x = pol.x / 2; pol.y = pol.y / 2; }
+            if (nx == 0 && ny == 0 && j0 + e == 0) pol = float2{0, 0};
+            const float2 d = v[e];
+            sp[e].x += pol.x * d.x - pol.y * d.y;
+            sp[e].y += pol.x * d.y + pol.y * d.x;
+            sn[e].x += pol.x * d.x + pol.y * d.y;
+            sn[e].y += pol.x * d.y - pol.y * d.x;
+        }
+    }
+    if (!ok) return;
+    const int64_t rho2 = (int64_t)nx * nx + (int64_t)ny * ny;
+    const double dw = g.dw;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int kz = j0 + e * TPT, nz = wrapn(kz, N);
+        const int64_t n2 = rho2 + (int64_t)nz * nz;
+        float cf, sf;
+        z_phase<float>(n2, g, cf, sf);
+        const double cq = cf, sq = sf;
+        const double2 SP = {(double)sp[e].x * dw, (double)sp[e].y * dw};
+        const double2 SN = {(double)sn[e].x * dw, (double)sn[e].y * dw};
+        float2* a = A + tile0 + (int64_t)kz * TX;
+        const float2 a11 = ld_stream(a), a12 = ld_stream(a + 2 * ms), a22 = ld_stream(a + 3 * ms);
+        st_stream(a, float2{(float)((double)a11.x + cq * SP.x), (float)((double)a11.y + cq * SP.y)});
+        st_stream(a + 3 * ms, float2{(float)((double)a22.x + sq * SN.x), (float)((double)a22.y + sq * SN.y)});
+        if (!g.fix_swap) {
+            const double2 r12 = {(double)a12.x + (sq * SP.x + cq * SN.x), (double)a12.y + (sq * SP.y + cq * SN.y)};
+            const double n6 = n2 > 0 ? ((double)rho2 / (double)n2) / 2 * dw : 0.0;
+            st_stream(a + 2 * ms, float2{(float)r12.x, (float)r12.y});
+            st_stream(a + ms, float2{(float)(r12.x - cq * (n6 * (double)v[e].x)), (float)(r12.y - cq * (n6 * (double)v[e].y))});
+        } else {
+            const float2 a21 = ld_stream(a + ms);
+            st_stream(a + ms, float2{(float)((double)a21.x + sq * SP.x), (float)((double)a21.y + sq * SP.y)});
+            st_stream(a + 2 * ms, float2{(float)((double)a12.x + cq * SN.x), (float)((double)a12.y + cq * SN.y)});
+        }
     }
 }
 
@@ -811,22 +936,6 @@ void launch_fft_rows(hipStream_t s, int N, void* data, int64_t nrows, const FftP
 // LDS when the update runs.  With fix_swap: A21 += s dw SP, A12 += c dw SN.
 
 constexpr int ZNT = 512;  // threads of the accumulation pass
-
-template <typename T>
-__device__ __forceinline__ void pol_vec(int nx, int ny, int nz, typename V2<T>::type* p)
-{
-    // grav_waves.f90:165-183 (n != 0)
-    T qx = (T)nx, qy = (T)ny, qz = (T)nz;
-    T q = sqrt(qx * qx + qy * qy + qz * qz);
-    qx = qx / q; qy = qy / q; qz = qz / q;
-    T r = sqrt(qx * qx + qy * qy);
-    T c, s;
-    if (r > 0) { c = qx / r; s = qy / r; }
-    else { c = 1; s = 0; }
-    p[0] = {qz * c, -s};
-    p[1] = {qz * s, c};
-    p[2] = {-r, 0};
-}
 
 template <typename T>
 __global__ void __launch_bounds__(ZNT) gw_zpass_acc_kernel(int N, int P, const typename V2<T>::type* __restrict__ W,
@@ -1016,6 +1125,11 @@ void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A
         constexpr int TXP = p2_ztx<T, NN>();
         if (!TiledLayout<NN, TXP>::matches(L))
             throw Error(AXG_EINVAL, "accumulation layout does not match the z pass tile");
+        if constexpr (sizeof(T) == 4 && P2<NN>::R9) {
+            hipLaunchKernelGGL((gw_zpass_p9_kernel<NN>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
+                               (const float2*)W, (float2*)A, (const float2*)tw, g, sr, lat);
+            return;
+        }
         if constexpr (p2_zpar<T, NN>()) {
             constexpr int NT = p2_zpar_threads<T, NN>();
             if ((int64_t)L.ntile * NN * nlat * (NT / 64) <= ZPAR_WAVES) {

@@ -144,7 +144,7 @@ void launch_kick_drift(hipStream_t s, int N, const void* phi_in, void* phi_out, 
 }
 
 
-// ------------------------------------------------------------------ fused pass for N = 2^L, 3 * 2^L
+// ------------------------------------------------------------------ fused pass for the compile-time sizes
 //
 // The same kick + source + drift, with the x transform of the three packed source planes
 // done in the same block (fft_p2.h): block = XR rows y at one z with one thread per site
@@ -168,7 +168,9 @@ template <int N> constexpr int fused_rows_wide() { return N >= 1024 ? 1 : (1024 
 // Multiplying by inv_d = 1/d2 gives the same bits when d2 is a power of two; for any other
 // dspa the host sets div and the FP64 path divides.  FP32 storage always multiplies: its
 // gradient is rounded to FP32, far coarser than the FP64 quotient's last bit.
-template <typename T>
+// EXS: sources formed in FP64 whatever the storage, as kick_drift_kernel forms them (the sizes with two
+// or more factors of three, whose FP32 accumulators have been made that way).
+template <typename T, bool EXS>
 __device__ __forceinline__ void kick_site(double2 c, double2 a1, double2 a2, double2 b1, double2 b2, double2 c1v,
                                           double2 c2v, double2& p, double2& f, typename V2<T>::type (&src)[3],
                                           const KickScalars& k, double inv_d, double d2, bool div,
@@ -189,7 +191,7 @@ __device__ __forceinline__ void kick_site(double2 c, double2 a1, double2 a2, dou
     p.x = k.f1 * p.x + k.f2 * lr + k.f3 * dr;
     p.y = k.f1 * p.y + k.f2 * li + k.f3 * di;
     f = double2{c.x + dt_drift * p.x, c.y + dt_drift * p.y};
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (sizeof(T) == 4 && !EXS) {
         // FP32 storage: the differences in FP64 (they cancel), the gradient and the products in
         // FP32, the precision the sources are stored in
         const float sx = (float)((a2.x - a1.x) * inv_d), sy = (float)((a2.y - a1.y) * inv_d);
@@ -303,7 +305,7 @@ __global__ void __launch_bounds__(XR * N) kick_source_xfft_kernel(
         double2 p = ldf<T, COMP>(pi, cpi, i);
         double2 f;
         T2 src[3];
-        kick_site<T>(c, a1, a2, b1, b2, c1v, c2v, p, f, src, k, inv_d, d2, div != 0, dt_drift);
+        kick_site<T, P2<N>::R9>(c, a1, a2, b1, b2, c1v, c2v, p, f, src, k, inv_d, d2, div != 0, dt_drift);
         stf<T, COMP>(pi, cpi, i, p);
         stf<T, COMP>(phi_out, cphi_out, i, f);
         s[rr * N + x] = src[0];
@@ -494,8 +496,8 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
         ld_pair<T, COMP, true>(pi, cpi, row + x0, p0, p1);
         double2 f0, f1;
         T2 sa[3], sb[3];
-        kick_site<T>(c0, l, c1, b10, b20, z10, z20, p0, f0, sa, k, inv_d, d2, div != 0, dt_drift);
-        kick_site<T>(c1, c0, r, b11, b21, z11, z21, p1, f1, sb, k, inv_d, d2, div != 0, dt_drift);
+        kick_site<T, P2<N>::R9>(c0, l, c1, b10, b20, z10, z20, p0, f0, sa, k, inv_d, d2, div != 0, dt_drift);
+        kick_site<T, P2<N>::R9>(c1, c0, r, b11, b21, z11, z21, p1, f1, sb, k, inv_d, d2, div != 0, dt_drift);
         st_pair<T, COMP, true>(pi, cpi, row + x0, p0, p1);
         st_pair<T, COMP, true>(phi_out, cphi_out, row + x0, f0, f1);
 #pragma unroll
@@ -634,6 +636,14 @@ bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi
     case 256: go.template operator()<256>(); break;
     case 512: go.template operator()<512>(); break;
     case 1024: go.template operator()<1024>(); break;
+    case 72: go.template operator()<72>(); break;
+    case 144: go.template operator()<144>(); break;
+    case 216: go.template operator()<216>(); break;
+    case 288: go.template operator()<288>(); break;
+    case 432: go.template operator()<432>(); break;
+    case 576: go.template operator()<576>(); break;
+    case 648: go.template operator()<648>(); break;
+    case 864: go.template operator()<864>(); break;
     case 24: go.template operator()<24>(); break;
     case 48: go.template operator()<48>(); break;
     case 96: go.template operator()<96>(); break;
