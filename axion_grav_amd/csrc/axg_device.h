@@ -277,13 +277,13 @@ __device__ __forceinline__ void philox4x32(uint32_t& c0, uint32_t& c1, uint32_t&
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
 #pragma unroll
     for (int r = 0; r < 10; r++) {
-        uint32_t h0 = __umulhi(M0, c0), l0 = M0 * c0;
-        uint32_t h1 = __umulhi(M1, c2), l1 = M1 * c2;
-        uint32_t n0 = h1 ^ c1 ^ k0, n2 = h0 ^ c3 ^ k1;
+        // one 64-bit product each (its two halves in one instruction)
+        const uint64_t p0 = (uint64_t)M0 * c0, p1 = (uint64_t)M1 * c2;
+        const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
         c0 = n0;
-        c1 = l1;
+        c1 = (uint32_t)p1;
         c2 = n2;
-        c3 = l0;
+        c3 = (uint32_t)p0;
         k0 += W0;
         k1 += W1;
     }
@@ -303,9 +303,10 @@ __device__ __forceinline__ void unit_gauss(uint64_t seed, uint32_t tag, uint32_t
     const double u1 = ((double)a + 1.0) / 9007199254740992.0;
     const double u2 = ((double)b + 1.0) / 9007199254740992.0;
     const double r = sqrt(-2.0 * log(u1));
-    const double th = 6.283185307179586 * u2;
-    re = r * cos(th);
-    im = r * sin(th);
+    double si, co;
+    sincos(6.283185307179586 * u2, &si, &co);
+    re = r * co;
+    im = r * si;
 }
 
 // ------------------------------------------------------------------ the reference's random stream

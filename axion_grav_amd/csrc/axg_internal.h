@@ -287,8 +287,25 @@ template <typename T, bool COMP>
 void launch_masked_field(hipStream_t s, int N, const void* pi, const void* cpi, const int8_t* flags,
                          double2* out, double fill_unmasked, bool use_pi);
 
+// Transforms of the field spectrum and its covariance (spectrum.hip).  They leave the folded power of
+// row (ky, kz): |.|^2 of kx = j and -j added, j = 0..N/2, as reals at the beginning of the row's N
+// complex values, which launch_spec_bin and launch_n2_hist read.  The first of each kind returns
+// false (nothing launched) where N has no compile-time kernels; lim != 0 or a finite n2max leaves
+// rows beyond n2max out.
+bool launch_spec_modes_x(hipStream_t s, int N, const Draws& dr, int iter, const uint16_t* bin_of_n2, int64_t n2max,
+                         const double* sigma, double2* out, const double2* tw);
+template <typename T, bool COMP>
+bool launch_spec_z_field(hipStream_t s, int N, const void* pi, const void* cpi, const int8_t* flags, double fill, bool use_pi,
+                         double2* out, const double2* tw);
+void launch_spec_y(hipStream_t s, int N, double2* data, int sign, int lim, int64_t n2max, const double2* tw);
+size_t spec_mask_bytes(int N);
+void launch_spec_mask_bits(hipStream_t s, int N, const int8_t* flags, uint8_t* bits);
+void launch_spec_z_mask(hipStream_t s, int N, double2* data, const uint8_t* bits, const double2* tw);
+void launch_spec_fold_x(hipStream_t s, int N, double2* data, int64_t n2max, double amp, const double2* tw);
+void launch_spec_fold(hipStream_t s, int N, double2* data, double amp);
+
 void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* bin_of_n2, int64_t n2max, int nb,
-                     double scale, double* partial, int nwg, double* out);
+                     double* partial, int nwg, double* out);
 
 void launch_n2_hist(hipStream_t s, int N, const double2* data, double* plane_part, double* hist);
 

@@ -202,6 +202,7 @@ struct axg_handle {
     double* d_cnt = nullptr;  // lattice points per n^2
     double* d_hist = nullptr;
     double* d_plane = nullptr;
+    uint8_t* d_maskbits = nullptr;  // the mask as a realisation's z transforms read it (spectrum.hip)
     // kernel timing
     bool prof = false;
     std::vector<hipEvent_t> ev;      // event pool
@@ -1485,6 +1486,29 @@ static void fft3d_work(axg_handle* h, double2* d, int sign = +1)
     }
 }
 
+// Folded power of the BACKWARD transform of (mask ? 0 : pi) or, use_pi false, of the window
+// (mask ? 0 : fill), times amp^2, into h->work; the rows beyond n2max are left out.
+template <typename T, bool COMP>
+static void masked_power(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
+{
+    const double2* tw = (const double2*)h->tw64;
+    if (launch_spec_z_field<T, COMP>(h->stream, h->N, h->pi, h->cpi, h->flags, fill, use_pi, h->work, tw)) {
+        launch_spec_y(h->stream, h->N, h->work, +1, n2max < h->nn2 - 1, n2max, tw);
+        launch_spec_fold_x(h->stream, h->N, h->work, n2max, amp, tw);
+        return;
+    }
+    launch_masked_field<T, COMP>(h->stream, h->N, h->pi, h->cpi, h->flags, h->work, fill, use_pi);
+    fft3d_work(h, h->work);
+    launch_spec_fold(h->stream, h->N, h->work, amp);
+}
+
+static void masked_power_any(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
+{
+    if (h->comp) masked_power<float, true>(h, use_pi, fill, amp, n2max);
+    else if (h->fp32) masked_power<float, false>(h, use_pi, fill, amp, n2max);
+    else masked_power<double, false>(h, use_pi, fill, amp, n2max);
+}
+
 // Runs body(lo, hi) over [0, n) split into contiguous ranges on up to 16 host threads (the
 // one-time spectrum tables: each index writes only its own outputs, so the split changes nothing).
 template <typename F> static void host_parallel(int64_t n, F&& body)
@@ -1582,9 +1606,7 @@ extern "C" int axg_field_spectrum(axg_handle* h, double tau, double* qmid, doubl
         const int ncov = nb * (nb + 1) / 2;
         const int nwg = 1024;
         // compute_matrix_deconv (spectrum.f90:358-433): window = dv_spa with mask cells zeroed
-        if (h->comp) launch_masked_field<float, true>(h->stream, h->N, nullptr, nullptr, h->flags, h->work, p.dv_spa, false);
-        else launch_masked_field<double, false>(h->stream, h->N, nullptr, nullptr, h->flags, h->work, p.dv_spa, false);
-        fft3d_work(h, h->work);
+        masked_power_any(h, false, p.dv_spa, 1.0, h->nn2 - 1);
         launch_n2_hist(h->stream, h->N, h->work, h->d_plane, h->d_hist);
         double* mat0 = h->red;
         double* tat0 = h->red + ncov;
@@ -1596,13 +1618,10 @@ extern "C" int axg_field_spectrum(axg_handle* h, double tau, double* qmid, doubl
         AXG_HIP(hipMemcpyAsync(t0.data(), tat0, ncov * 8, hipMemcpyDeviceToHost, h->stream));
         AXG_HIP(hipStreamSynchronize(h->stream));
         // compute_conv_spec (spectrum.f90:474-563): masked pi -> FFT -> *dv_spa -> binned
-        if (h->comp) launch_masked_field<float, true>(h->stream, h->N, h->pi, h->cpi, h->flags, h->work, 0.0, true);
-        else if (h->fp32) launch_masked_field<float, false>(h->stream, h->N, h->pi, nullptr, h->flags, h->work, 0.0, true);
-        else launch_masked_field<double, false>(h->stream, h->N, h->pi, nullptr, h->flags, h->work, 0.0, true);
-        fft3d_work(h, h->work);
+        masked_power_any(h, true, 0.0, p.dv_spa, h->spec_n2max);
         double* out = h->red + (size_t)nwg * 2 * nb;
         require((size_t)(nwg + 1) * 2 * nb * 8 <= h->red_bytes, "reduction scratch too small");
-        launch_spec_bin(h->stream, h->N, h->work, h->spec_bin, h->spec_n2max, nb, p.dv_spa, h->red, nwg, out);
+        launch_spec_bin(h->stream, h->N, h->work, h->spec_bin, h->spec_n2max, nb, h->red, nwg, out);
         std::vector<double> r(2 * nb);
         AXG_HIP(hipMemcpyAsync(r.data(), out, 2 * nb * 8, hipMemcpyDeviceToHost, h->stream));
         AXG_HIP(hipStreamSynchronize(h->stream));
@@ -1712,12 +1731,25 @@ extern "C" int axg_field_covariance(axg_handle* h, uint64_t seed, int32_t min_mc
         int iter = 1;
         bool converged = false;
         const Draws dr = h->draws((uint32_t)seed, (uint32_t)(seed >> 32));
+        if (p2_size(N)) {
+            if (!h->d_maskbits) h->d_maskbits = (uint8_t*)h->alloc(spec_mask_bytes(N));
+            launch_spec_mask_bits(h->stream, N, h->flags, h->d_maskbits);
+        }
         for (; iter <= max_mc; iter++) {
-            launch_cov_modes(h->stream, N, dr, iter, h->spec_bin, d_sig, h->work);
-            fft3d_work(h, h->work, -1);
-            launch_mask_zero(h->stream, h->n3, h->flags, h->work);
-            fft3d_work(h, h->work, +1);
-            launch_spec_bin(h->stream, N, h->work, h->spec_bin, h->spec_n2max, nb, 1.0, part, nwg, out);
+            const double2* tw = (const double2*)h->tw64;
+            if (launch_spec_modes_x(h->stream, N, dr, iter, h->spec_bin, h->spec_n2max, d_sig, h->work, tw)) {
+                launch_spec_y(h->stream, N, h->work, -1, 1, h->spec_n2max, tw);
+                launch_spec_z_mask(h->stream, N, h->work, h->d_maskbits, tw);
+                launch_spec_y(h->stream, N, h->work, +1, 1, h->spec_n2max, tw);
+                launch_spec_fold_x(h->stream, N, h->work, h->spec_n2max, 1.0, tw);
+            } else {
+                launch_cov_modes(h->stream, N, dr, iter, h->spec_bin, d_sig, h->work);
+                fft3d_work(h, h->work, -1);
+                launch_mask_zero(h->stream, h->n3, h->flags, h->work);
+                fft3d_work(h, h->work, +1);
+                launch_spec_fold(h->stream, N, h->work, 1.0);
+            }
+            launch_spec_bin(h->stream, N, h->work, h->spec_bin, h->spec_n2max, nb, part, nwg, out);
             AXG_HIP(hipMemcpyAsync(r.data(), out, 2 * nb * 8, hipMemcpyDeviceToHost, h->stream));
             AXG_HIP(hipStreamSynchronize(h->stream));
             // pow = mat_deconv pow0 - power (dspmv with beta = 1, spectrum.f90:675-677)

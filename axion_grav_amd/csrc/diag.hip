@@ -5,6 +5,8 @@
 // deterministic: fixed per-block partial order, then a fixed-order sum over blocks.
 #include "axg_internal.h"
 
+#include <algorithm>
+
 namespace axg {
 
 constexpr int RED_NT = 256;
@@ -417,106 +419,135 @@ void launch_masked_field(hipStream_t s, int N, const void* pi, const void* cpi, 
     AXG_HIP(hipGetLastError());
 }
 
-// Shell binning over the full spectrum (spectrum.f90:530-556).  Row (ky,kz) is folded onto
-// j = |nx| = 0..N/2 (kx = j and kx = N-j), along which the bin is non-decreasing, then every
-// run of equal bins is summed by the thread at its start (same deterministic scheme as the
-// GW binning).  pow[b] += |d*amp|^2 (times dv_wav on the host), num[b] += 1 per mode.
-// As in the GW binning, each thread loads its values of the next row while the current row is
-// binned (only modes up to the last bin's |n|^2, without waiting for the bin lookup), and each run
-// is summed over the length its last element recorded; the sums and their order are unchanged.
-constexpr int SPEC_BIN_NT = 256, SPEC_BIN_KPT = 3;  // folded j values per thread: N / 2 + 1 <= 768
+// Shell binning over the full spectrum (spectrum.f90:530-556) of the folded power (axg_internal.h): row
+// (ky,kz) holds j = |nx| = 0..N/2, along which the bin is non-decreasing, so every bin is one run
+// of the row.  pow[b] += |.|^2 (times dv_wav on the host), num[b] += 1 per mode.
+//
+// A wave takes a row at a time, into its own LDS bins: the last element of a run records where the run
+// ends and the lane at its start sums it in order.  No barrier and no other wave is waited for
+// (one row per 256-thread block, three barriers each, took 122 us at 256^3 and 640 us at 512^3
+// where the reads need 10 and 70).  The waves' bins are added in order at the end, and the blocks'
+// by sum_columns: the reduction is deterministic.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
-__global__ void __launch_bounds__(SPEC_BIN_NT) spec_bin_kernel(int N, const double2* __restrict__ d,
-                                                               const uint16_t* __restrict__ bin_of_n2, int64_t n2max,
-                                                               int nb, double amp, double* __restrict__ partial)
+// LDS of one wave: 2 nb bins and N/2 + 1 values in FP64, then the values' bins and the runs' ends
+static size_t spec_bin_lds(int N, int nb)
+{
+    return ((size_t)(2 * nb + N / 2 + 1) * sizeof(double) + (size_t)(N / 2 + 1 + nb) * sizeof(int) + 7) / 8 * 8;
+}
+
+template <int KP>
+__global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __restrict__ d,
+                                                       const uint16_t* __restrict__ bin_of_n2, int64_t n2max, int nb,
+                                                       double* __restrict__ partial)
 {
     extern __shared__ double sh[];
-    double* bins = sh;
-    double* v = sh + 2 * nb;
-    double* cnt = v + (N / 2 + 1);
-    int* bb = (int*)(cnt + (N / 2 + 1));
-    int* rend = bb + (N / 2 + 1);  // nb: one past the last j of bin b's run in the row
-    const int nh = N / 2 + 1;
+    const int nh = N / 2 + 1, lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int per = 2 * nb + nh + (nh + nb + 1) / 2;
+    double* bins = sh + (size_t)w * per;
+    double* v = bins + 2 * nb;
+    int* bb = (int*)(v + nh);
+    int* rend = bb + nh;  // nb: one past the last j of bin b's run in the row
     const int64_t NN = (int64_t)N * N;
-    for (int b = threadIdx.x; b < 2 * nb; b += blockDim.x) bins[b] = 0;
-    double2 a[SPEC_BIN_KPT], e[SPEC_BIN_KPT];
-    int bq[SPEC_BIN_KPT];
+    for (int b = lane; b < 2 * nb; b += 64) bins[b] = 0;
+    double a[KP];
+    int bq[KP];
+    const int64_t step = (int64_t)gridDim.x * nw;
+    // the wave's next row with a binned mode, its values and bins in registers
     auto fetch = [&](int64_t row) {
-        const int kz = (int)(row / N), ky = (int)(row - (int64_t)kz * N);
-        const int ny = wrapn(ky, N), nz = wrapn(kz, N);
-        const double2* r = d + row * N;
+        for (; row < NN; row += step) {
+            const int kz = (int)(row / N), ky = (int)(row - (int64_t)kz * N);
+            const int ny = wrapn(ky, N), nz = wrapn(kz, N);
+            const int64_t m2 = (int64_t)ny * ny + (int64_t)nz * nz;
+            if (m2 > n2max) continue;
+            const double* r = (const double*)(d + row * N);
 #pragma unroll
-        for (int i = 0; i < SPEC_BIN_KPT; i++) {
-            const int j = threadIdx.x + i * SPEC_BIN_NT;
-            if (j < nh) {
-                const int64_t n2 = (int64_t)j * j + (int64_t)ny * ny + (int64_t)nz * nz;
-                bq[i] = bin_of_n2[n2];
-                if (n2 <= n2max) {
-                    a[i] = r[j];
-                    if (j > 0 && j < N / 2) e[i] = r[N - j];
-                }
+            for (int i = 0; i < KP; i++) {
+                const int j = lane + i * 64;
+                const int64_t n2 = (int64_t)j * j + m2;
+                const bool in = j < nh && n2 <= n2max;
+                bq[i] = in ? bin_of_n2[n2] : 0;
+                a[i] = in ? r[j] : 0.0;
             }
+            break;
         }
+        return row;
     };
-    int64_t row = blockIdx.x;
-    if (row < NN) fetch(row);
-    __syncthreads();
-    for (; row < NN; row += gridDim.x) {
+    int64_t row = fetch((int64_t)blockIdx.x * nw + w);
+    while (row < NN) {
 #pragma unroll
-        for (int i = 0; i < SPEC_BIN_KPT; i++) {
-            const int j = threadIdx.x + i * SPEC_BIN_NT;
+        for (int i = 0; i < KP; i++) {
+            const int j = lane + i * 64;
             if (j < nh) {
-                double s = 0, c = 0;
-                if (bq[i] > 0) {
-                    double ax = a[i].x * amp, ay = a[i].y * amp;
-                    s = ax * ax + ay * ay;
-                    c = 1;
-                    if (j > 0 && j < N / 2) {
-                        double ex = e[i].x * amp, ey = e[i].y * amp;
-                        s += ex * ex + ey * ey;
-                        c = 2;
-                    }
-                }
-                v[j] = s;
-                cnt[j] = c;
+                v[j] = a[i];
                 bb[j] = bq[i];
             }
         }
-        if (row + gridDim.x < NN) fetch(row + gridDim.x);
-        __syncthreads();
-        for (int j = threadIdx.x; j < nh; j += blockDim.x) {
-            const int b = bb[j];
-            if (b > 0 && (j == nh - 1 || bb[j + 1] != b)) rend[b - 1] = j + 1;
-        }
-        __syncthreads();
-        for (int j = threadIdx.x; j < nh; j += blockDim.x) {
-            int b = bb[j];
-            if (b > 0 && (j == 0 || bb[j - 1] != b)) {
-                const int end = rend[b - 1];
-                double sn = 0, sd = 0;
-                for (int k = j; k < end; k++) { sn += v[k]; sd += cnt[k]; }
-                bins[b - 1] += sn;
-                bins[nb + b - 1] += sd;
+        row = fetch(row + step);
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < KP; i++) {
+            const int j = lane + i * 64;
+            if (j < nh) {
+                const int b = bb[j];
+                if (b > 0 && (j == nh - 1 || bb[j + 1] != b)) rend[b - 1] = j + 1;
             }
         }
-        __syncthreads();
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < KP; i++) {
+            const int j = lane + i * 64;
+            if (j < nh) {
+                const int b = bb[j];
+                if (b > 0 && (j == 0 || bb[j - 1] != b)) {
+                    const int end = rend[b - 1];
+                    double sn = 0;
+#pragma unroll 4
+                    for (int k = j; k < end; k++) sn += v[k];
+                    bins[b - 1] += sn;
+                    // two modes for each j, one for j = 0 and N/2
+                    bins[nb + b - 1] += (double)(2 * (end - j) - (j == 0) - (end == nh));
+                }
+            }
+        }
+        wave_lds_sync();
     }
-    for (int b = threadIdx.x; b < 2 * nb; b += blockDim.x) partial[(int64_t)blockIdx.x * 2 * nb + b] = bins[b];
+    __syncthreads();
+    for (int b = threadIdx.x; b < 2 * nb; b += blockDim.x) {
+        double t = 0;
+        for (int k = 0; k < nw; k++) t += sh[(size_t)k * per + b];
+        partial[(int64_t)blockIdx.x * 2 * nb + b] = t;
+    }
 }
 
 void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* bin_of_n2, int64_t n2max, int nb,
-                     double scale, double* partial, int nwg, double* out)
+                     double* partial, int nwg, double* out)
 {
-    int nh = N / 2 + 1;
-    if (nh > SPEC_BIN_KPT * SPEC_BIN_NT) throw Error(AXG_EINVAL, "field spectrum: N too large for the binning kernel");
-    size_t lds = (size_t)(2 * nb + 2 * nh) * sizeof(double) + (size_t)(nh + nb) * sizeof(int);
-    hipLaunchKernelGGL(spec_bin_kernel, dim3(nwg), dim3(SPEC_BIN_NT), lds, s, N, data, bin_of_n2, n2max, nb, scale,
-                       partial);
+    const int kp = (N / 2 + 1 + 63) / 64;
+    if (kp > 9) throw Error(AXG_EINVAL, "field spectrum: N too large for the binning kernel");
+    // four waves a block, fewer where their bins pass 64 KiB
+    const size_t per = spec_bin_lds(N, nb);
+    const int nw = (int)std::max<size_t>(1, std::min<size_t>(4, 65536 / per));
+    auto go = [&]<int KP>() {
+        hipLaunchKernelGGL(spec_bin_kernel<KP>, dim3(nwg), dim3(64 * nw), per * nw, s, N, data, bin_of_n2, n2max, nb, partial);
+    };
+    if (kp <= 1) go.template operator()<1>();
+    else if (kp == 2) go.template operator()<2>();
+    else if (kp == 3) go.template operator()<3>();
+    else if (kp == 4) go.template operator()<4>();
+    else if (kp == 5) go.template operator()<5>();
+    else if (kp <= 7) go.template operator()<7>();
+    else go.template operator()<9>();
     AXG_HIP(hipGetLastError());
     sum_columns(s, partial, nwg, 2 * nb, out);
 }
 
-// Histogram of |W|^2 by n^2 = |n|^2, deterministic: block kz walks its plane by a = |ny|
+// Histogram of |W|^2 (its folded power) by n^2 = |n|^2, deterministic: block kz walks its plane by a = |ny|
 // (a = 0 .. N/2, in order).  The rows ky = a and ky = N - a share a, so their values at each
 // folded j = |nx| land on the same m = j^2 + a^2 and are added together first; within one a the
 // j hit distinct m, so the per-plane partial plane[kz][m] needs no atomics.  Each thread loads
@@ -532,22 +563,17 @@ __global__ void __launch_bounds__(N2P_NT) n2_plane_kernel(int N, const double2* 
     const int kz = blockIdx.x;
     double* pp = plane + (int64_t)kz * mm;
     for (int64_t m = threadIdx.x; m < mm; m += blockDim.x) pp[m] = 0;
-    double2 u[N2P_KPT][4];  // rows a and N - a, each at j and N - j
+    double u[N2P_KPT][2];  // rows a and N - a
     auto fetch = [&](int a) {
-        const double2* r1 = d + ((int64_t)kz * N + a) * N;
-        const double2* r2 = d + ((int64_t)kz * N + (N - a)) * N;
+        const double* r1 = (const double*)(d + ((int64_t)kz * N + a) * N);
+        const double* r2 = (const double*)(d + ((int64_t)kz * N + (N - a)) * N);
         const bool two = a > 0 && a < N / 2;
 #pragma unroll
         for (int i = 0; i < N2P_KPT; i++) {
             const int j = threadIdx.x + i * N2P_NT;
             if (j < nh) {
-                const bool mir = j > 0 && j < N / 2;
                 u[i][0] = r1[j];
-                if (mir) u[i][1] = r1[N - j];
-                if (two) {
-                    u[i][2] = r2[j];
-                    if (mir) u[i][3] = r2[N - j];
-                }
+                if (two) u[i][1] = r2[j];
             }
         }
     };
@@ -558,16 +584,7 @@ __global__ void __launch_bounds__(N2P_NT) n2_plane_kernel(int N, const double2* 
         double s[N2P_KPT];
 #pragma unroll
         for (int i = 0; i < N2P_KPT; i++) {
-            const int j = threadIdx.x + i * N2P_NT;
-            const bool mir = j > 0 && j < N / 2;
-            double t = u[i][0].x * u[i][0].x + u[i][0].y * u[i][0].y;
-            if (mir) t += u[i][1].x * u[i][1].x + u[i][1].y * u[i][1].y;
-            if (two) {
-                double t2 = u[i][2].x * u[i][2].x + u[i][2].y * u[i][2].y;
-                if (mir) t2 += u[i][3].x * u[i][3].x + u[i][3].y * u[i][3].y;
-                t += t2;
-            }
-            s[i] = t;
+            s[i] = two ? u[i][0] + u[i][1] : u[i][0];
         }
         if (a < N / 2) fetch(a + 1);
 #pragma unroll

@@ -592,6 +592,9 @@ template <typename T, int N> constexpr int p2_tx()
     return tx;
 }
 
+// Rows a block of the row passes takes, with N/8 threads each.
+template <int N> constexpr int p2_rows_per_block() { return (N / 8) >= 256 ? 1 : 256 / (N / 8); }
+
 // Runs F.template operator()<N>() for the sizes of p2_size; returns false otherwise.
 template <typename F> bool p2_dispatch(int N, F&& f)
 {

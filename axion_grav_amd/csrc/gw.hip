@@ -879,8 +879,6 @@ __global__ void __launch_bounds__(FFT_NT) fft_rows_kernel(int N, int TB, int64_t
 
 // Rows of the compile-time sizes: RB rows per block of RB * N/8 threads, each thread holding 8 elements of its
 // row in registers (fft_p2.h), loads and stores coalesced along the row.
-template <int N> constexpr int p2_rows_per_block() { return (N / 8) >= 256 ? 1 : 256 / (N / 8); }
-
 template <typename T, int N, int SIGN>
 __global__ void __launch_bounds__(p2_rows_per_block<N>() * (N / 8))
     fft_rows_p2_kernel(typename V2<T>::type* __restrict__ data, int64_t nrows, const typename V2<T>::type* __restrict__ tw)
