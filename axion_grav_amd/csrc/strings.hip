@@ -9,13 +9,17 @@
 // lives in registers: the insertion of a start point and the bubble sort are unrolled over the
 // five simplex slots, so no index into them depends on data.
 //
-// Two stages, because the simplex phase diverges: most fits converge within a few iterations,
+// The random starts have a kernel of their own with eight lanes per string (fit_starts): the simplex needs a
+// string's best five only, and one lane's 1001 chi2 were most of the fit's time on lattices whose
+// strings do not fill the chip twice over (256^3: 94,000).
+//
+// The simplex takes two kernels, because it diverges: most fits converge within a few iterations,
 // but about one string in seven never reaches chi2 <= 0.05 and runs all 1000, so nearly every
-// wave of 64 strings would wait for 1000 iterations while most of its lanes idle.  Stage one
-// runs the random starts and the first `split` simplex iterations of every string; a string still
-// searching then parks its simplex (5 points, 5 chi2, iteration count) in a list.  Stage two
-// continues the parked strings, one per thread, so the long searches share waves.  A string's
-// search is the same sequence of operations whichever stage ends it, so the records do not
+// wave of 64 strings would wait for 1000 iterations while most of its lanes idle.  The first
+// runs the first `split` simplex iterations of every string; a string still
+// searching then puts its simplex (5 points, 5 chi2, iteration count) back and itself on a list.  The
+// second continues the listed strings, one per thread, so the long searches share waves.  A string's
+// search is the same sequence of operations whichever kernel ends it, so the records do not
 // depend on `split`.  The per-block sums are taken afterwards from the records.
 //
 // Within a wave the simplex iterations run in lockstep, and a shrink (four chi2) on any lane
@@ -70,8 +74,12 @@ struct Phases {
 __device__ __noinline__ double chi2_string_v(Phases ph, double p0, double p1, double p2, double p3)
 {
 #pragma clang fp contract(off)
-    double mu = p0, phi = p1, u0 = p2 * cos(p3), v0 = p2 * sin(p3);
-    double cm = mu, sm = sqrt(1.0 - mu * mu), cp = cos(phi), sp = sin(phi);
+    // (a sine and a cosine share their argument's reduction: 1440 -> 1206 VALU instructions, same bits)
+    double ct, st, cp, sp;
+    sincos(p3, &st, &ct);
+    sincos(p1, &sp, &cp);
+    double mu = p0, u0 = p2 * ct, v0 = p2 * st;
+    double cm = mu, sm = sqrt(1.0 - mu * mu);
     double a = 0, b = 0;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -182,62 +190,197 @@ __device__ __forceinline__ void copy4(double* d, const double* s)
 // the five simplex points p and their chi2 c2.
 constexpr double STR_TOL = 0.05;  // chi2 at which the simplex stops
 
-// 1001 random starts keep the best five (the first two unsorted, as in the reference).
-// The search arrays are locals here and copied out at the end: with the caller's arrays
-// (references) the compiler moved c2 to scratch memory inside the 1001-start loop.
-__device__ __forceinline__ void fit_starts(const Phases& ph, const Draws& dr, int64_t s,
-                                           double (&p_out)[NSIMP + 1][4], double (&c2_out)[NSIMP + 1])
+// The random starts, eight lanes (an octet) per string.  1001 starts keep the best five (the first two
+// unsorted, as in the reference); about 30 of them ever get into the five, and the chi2 of the others is
+// not used.  So each start is first estimated in FP32 (start_estimate, a fifth of the FP64 chi2's
+// instructions), eight starts of the string at once, and one whose estimate exceeds what the five can
+// still take by more than the estimate's error is passed over.  The rest wait in the octet's queue;
+// their FP64 chi2 are evaluated eight at a time and inserted in start order.  The five and their
+// chi2 are the same bit for bit.  Kernel with the first 32 simplex iterations of every string, 512^3,
+// 761,000 strings: 30 -> 12.1 + 2.4 ms; 256^3, 94,000: 5.9 -> 2.4 + 0.5; 64^3, 1,400: 3.8 -> 0.6 + 0.4.
+
+constexpr int OCT = 8, START_Q = 16;  // lanes per string; starts an octet's queue holds
+// Above any error of start_estimate: with every corner farther than START_R from the line its angle is off by
+// less than 2 * 2e-6 / START_R + 3e-6 = 2.1e-4 (sine and cosine are good to 1.6e-7, the coordinates to
+// 2e-6), so the variance of the eight differences (each below 2 pi) by less than 2 * 2 pi * 2.1e-4 =
+// 2.7e-3, and FP32 sums add 1e-4.
+constexpr float START_R = 0.02f, START_EPS = 6e-3f;
+
+// atan2 to 2e-6: the ratio of the smaller to the larger, an odd polynomial for arctan on [0, 1] (least maximum
+// error fit, 1.6e-06), and the octant.
+__device__ __forceinline__ float atan2_near(float y, float x)
+{
+    const float ax = fabsf(x), ay = fabsf(y);
+    const float t = fminf(ax, ay) * __builtin_amdgcn_rcpf(fmaxf(ax, ay)), z = t * t;
+    float p = fmaf(fmaf(fmaf(fmaf(fmaf(-0.0117191039f, z, 0.0526472703f), z, -0.116426408f), z, 0.19354035f), z, -0.332622826f), z, 0.999977231f) * t;
+    p = ay > ax ? 1.57079633f - p : p;
+    p = x < 0 ? 3.14159265f - p : p;
+    return copysignf(p, y);
+}
+
+// chi2_string of the start with uniforms u (v = 1 - u) in FP32, or a value below zero where it may be off by more
+// than START_EPS: a corner nearer than START_R to the line, or a difference within 1e-3 of the wrap
+// at +-pi.
+__device__ __forceinline__ float start_estimate(const float (&ph)[8], const float (&u)[4], float v0)
+{
+    const float mu = 2 * u[0] - 1, sm = 2 * __builtin_amdgcn_sqrtf(u[0] * v0);
+    const float sp = __builtin_amdgcn_sinf(u[1] - 0.5f), cp = __builtin_amdgcn_cosf(u[1] - 0.5f);
+    const float rho = 0.866025404f * u[2];
+    const float cu = rho * __builtin_amdgcn_cosf(u[3] - 0.5f), cv = rho * __builtin_amdgcn_sinf(u[3] - 0.5f);
+    const float hx = 0.5f * mu * cp, hy = 0.5f * mu * sp, hz = 0.5f * sm, gx = 0.5f * sp, gy = 0.5f * cp;
+    float a = 0, b = 0, rmin = 1e9f, dmax = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float du = -cu + ((i & 1) ? hx : -hx) + ((i & 2) ? hy : -hy) - ((i & 4) ? hz : -hz);
+        const float dv = -cv - ((i & 1) ? gx : -gx) + ((i & 2) ? gy : -gy);
+        float d = ph[i] - atan2_near(dv, du);
+        d = d - 6.28318531f * rintf(d * 0.159154943f);
+        rmin = fminf(rmin, fmaxf(fabsf(du), fabsf(dv)));
+        dmax = fmaxf(dmax, fabsf(d));
+        a = fmaf(d, d, a);
+        b = b + d;
+    }
+    b = b * 0.125f;
+    const float c = fmaf(a, 0.125f, -(b * b));
+    return rmin < START_R || dmax > 3.1405f ? -1.0f : c;
+}
+
+// The four uniforms of start i in FP32 and 1 - the first; the stream's state xs moves on by its four draws.
+__device__ __forceinline__ void uniforms_near(const Draws& dr, uint64_t& xs, int64_t s, int i, float (&u)[4], float& v0)
+{
+    if (dr.mcg) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const double x = mcg59_u(xs);
+            u[k] = (float)x;
+            if (k == 0) v0 = (float)(1.0 - x);
+            xs = mcg59_next(xs);
+        }
+        return;
+    }
+    uint32_t c0 = (uint32_t)i, c1 = (uint32_t)s, c2 = (uint32_t)((uint64_t)s >> 32), c3 = 0x73747267u;
+    philox4x32(c0, c1, c2, c3, dr.k0, dr.k1);
+    const float sc = 2.3283064365386963e-10f, h = 0.5f * sc;  // 2^-32
+    u[0] = fmaf((float)c0, sc, h);
+    v0 = fmaf((float)~c0, sc, h);
+    u[1] = fmaf((float)c1, sc, h);
+    u[2] = fmaf((float)c2, sc, h);
+    u[3] = fmaf((float)c3, sc, h);
+}
+
+// What the next start is compared with once m waiting starts are in, at most: each of them replaces c2[NSIMP] by
+// itself or by the slot before.  (The first two starts are not sorted, so a slot can hold more than the
+// one after it, and move up.)
+__device__ __forceinline__ double start_limit(const double (&c2)[NSIMP + 1], int m)
+{
+    double lim = c2[NSIMP];
+#pragma unroll
+    for (int j = 1; j <= NSIMP; j++)
+        if (m >= j) lim = fmax(lim, c2[NSIMP - j]);
+    return lim;
+}
+
+// Start t with its chi2 into the five (n0 + 1 of them are filled; n0 = -1 at first).
+__device__ __forceinline__ void insert_start(double (&p)[NSIMP + 1][4], double (&c2)[NSIMP + 1], int& n0, double chi2,
+                                             const double (&t)[4])
+{
+    if (n0 <= 0) {
+        n0 = n0 + 1;
+        if (n0 == 0) { c2[0] = chi2; copy4(p[0], t); }
+        else { c2[1] = chi2; copy4(p[1], t); }
+        return;
+    }
+    n0 = n0 + 1 < NSIMP ? n0 + 1 : NSIMP;
+    // insertion from slot n0 downwards: shift while chi2 <= the slot above
+    bool placed = false;
+#pragma unroll
+    for (int j = NSIMP; j >= 1; j--) {
+        if (j <= n0 && !placed) {
+            if (chi2 <= c2[j - 1]) {
+                c2[j] = c2[j - 1];
+                copy4(p[j], p[j - 1]);
+            } else {
+                c2[j] = chi2;
+                copy4(p[j], t);
+                placed = true;
+            }
+        }
+    }
+    if (!placed) { c2[0] = chi2; copy4(p[0], t); }
+}
+
+// The first stage of position_string for string s of an octet's eight lanes (o = 0..7); all lanes end with the
+// same five.  Every lane of the wave calls it (valid false: no string, only the votes).
+__device__ __forceinline__ void fit_starts(const Phases& ph, const Draws& dr, int64_t s, bool valid,
+                                           uint16_t (&queue)[64 / OCT][START_Q], double (&p)[NSIMP + 1][4],
+                                           double (&c2)[NSIMP + 1])
 {
 #pragma clang fp contract(off)
-    uint64_t xs = dr.mcg ? mcg59_jump(dr.x0, dr.pos + 4004 * (uint64_t)s) : 0;
     const double mx[4] = {1.0, PI_T, 0.86602540378443865, PI_T};
     const double mn[4] = {-1.0, -PI_T, 0.0, -PI_T};
-    double p[NSIMP + 1][4], c2[NSIMP + 1], t[4];
+    const int lane = (int)(threadIdx.x & 63), o = lane & (OCT - 1), g = lane / OCT;
+    const uint64_t xs0 = dr.mcg ? mcg59_jump(dr.x0, dr.pos + 4004 * (uint64_t)s) : 0;
+    constexpr uint64_t STEP = [] {  // what eight starts of four draws advance the stream by
+        uint64_t r = 1;
+        for (int i = 0; i < 4 * OCT; i++) r *= MCG59_A;
+        return r;
+    }();
+    uint64_t xs = dr.mcg ? mcg59_jump(xs0, 4 * (uint64_t)o) : 0;
 #pragma unroll
     for (int j = 0; j <= NSIMP; j++) {
         c2[j] = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) p[j][k] = 0;
     }
-    int n0 = -1;
-    for (int i = 0; i <= MAXIT; i++) {
-        double x[4];
-        uniforms(dr, xs, s, i, x);
+    float phf[8];
 #pragma unroll
-        for (int k = 0; k < 4; k++) t[k] = mx[k] * x[k] + mn[k] * (1 - x[k]);
-        double chi2 = chi2_string(ph, t);
-        if (n0 <= 0) {
-            n0 = n0 + 1;
-            if (n0 == 0) { c2[0] = chi2; copy4(p[0], t); }
-            else { c2[1] = chi2; copy4(p[1], t); }
-            continue;
+    for (int c = 0; c < 8; c++) phf[c] = (float)ph.v[c];
+    int n0 = -1, cnt = 0;
+    for (int i0 = 0; i0 <= MAXIT; i0 += OCT) {
+        const int i = i0 + o;
+        float u[4], v0;
+        uint64_t x = xs;
+        uniforms_near(dr, x, s, i, u, v0);
+        xs = (xs * STEP) & MCG59_MASK;
+        bool keep = valid && i <= MAXIT;
+        if (i0 > 0) {  // the first eight all go in
+            const float est = start_estimate(phf, u, v0) - START_EPS;
+            keep = keep && !(est > (float)start_limit(c2, NSIMP));
+            // starts of the octet before this one that may be in by then
+            const uint32_t before = (uint32_t)(__ballot(keep) >> (lane & ~(OCT - 1))) & ((1u << o) - 1);
+            keep = keep && !(est > (float)start_limit(c2, cnt + __popc(before)));
         }
-        // c2[n0] by selects (n0 is 1..NSIMP here), so that c2 stays in registers
-        double cn = n0 == 1 ? c2[1] : n0 == 2 ? c2[2] : n0 == 3 ? c2[3] : c2[4];
-        if (n0 < NSIMP || chi2 <= cn) {
-            n0 = n0 + 1 < NSIMP ? n0 + 1 : NSIMP;
-            // insertion from slot n0 downwards: shift while chi2 <= the slot above
-            bool placed = false;
+        const uint32_t kept = (uint32_t)(__ballot(keep) >> (lane & ~(OCT - 1))) & ((1u << OCT) - 1);
+        if (keep) queue[g][cnt + __popc(kept & ((1u << o) - 1))] = (uint16_t)i;
+        cnt += __popc(kept);
+        // evaluate the waiting starts: a round of eight is together, the first ones, the end, or a larger
+        // value is about to reach the last slot
+        const bool want = cnt >= OCT || i0 + OCT > MAXIT || (cnt > 0 && start_limit(c2, cnt) > c2[NSIMP]);
+        if (!__any(want)) continue;
+        __syncthreads();
+        for (int r = 0; __any(r < cnt); r += OCT) {
+            double chi2 = 0, t[4] = {0, 0, 0, 0};
+            if (r + o < cnt) {
+                const int iq = queue[g][r + o];
+                uint64_t xq = dr.mcg ? mcg59_jump(xs0, 4 * (uint64_t)iq) : 0;
+                double w[4];
+                uniforms(dr, xq, s, iq, w);
 #pragma unroll
-            for (int j = NSIMP; j >= 1; j--) {
-                if (j <= n0 && !placed) {
-                    if (chi2 <= c2[j - 1]) {
-                        c2[j] = c2[j - 1];
-                        copy4(p[j], p[j - 1]);
-                    } else {
-                        c2[j] = chi2;
-                        copy4(p[j], t);
-                        placed = true;
-                    }
-                }
+                for (int k = 0; k < 4; k++) t[k] = mx[k] * w[k] + mn[k] * (1 - w[k]);
+                chi2 = chi2_string(ph, t);
             }
-            if (!placed) { c2[0] = chi2; copy4(p[0], t); }
-        }
-    }
+            for (int k = 0; k < OCT; k++) {
+                const double ck = __shfl(chi2, k, OCT);
+                const bool in = r + k < cnt && (n0 < NSIMP || ck <= c2[NSIMP]);
+                if (!__any(in)) continue;
+                double tk[4];
 #pragma unroll
-    for (int j = 0; j <= NSIMP; j++) {
-        c2_out[j] = c2[j];
-        copy4(p_out[j], p[j]);
+                for (int kk = 0; kk < 4; kk++) tk[kk] = __shfl(t[kk], k, OCT);
+                if (in) insert_start(p, c2, n0, ck, tk);
+            }
+        }
+        __syncthreads();
+        cnt = 0;
     }
 }
 
@@ -373,6 +516,55 @@ __device__ __forceinline__ void fit_simplex(const Phases& ph, double (&p)[NSIMP 
         }
         shrink_chi2(L, shr, ph, p, c2);
         if (act) sort_simplex(p, c2);
+    }
+}
+
+// The same iterations with the eight lanes of an octet per string, all holding its simplex: the reflection,
+// expansion, contraction and four shrunk points are evaluated at once, one per lane, and the chi2 that
+// the iteration turns out to need are taken.  One chi2 round an iteration instead of up to six; of
+// the values, those that fit_simplex computes.
+__device__ __forceinline__ void fit_simplex_oct(const Phases& ph, double (&p)[NSIMP + 1][4], double (&c2)[NSIMP + 1], bool valid)
+{
+#pragma clang fp contract(off)
+    const double chi2max = 8 * PI_T * PI_T;
+    const int o = (int)(threadIdx.x & (OCT - 1));
+    double c[4], t[4], se[4], sc[4], q[4];
+    for (int it = 0; it < MAXIT; it++) {
+        const bool act = valid && c2[0] > STR_TOL;
+        if (!__any(act)) break;
+        centroid(p, c);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            t[k] = 2 * c[k] - p[NSIMP][k];
+            se[k] = 3 * c[k] - 4 * p[NSIMP][k];
+            sc[k] = 1.5 * c[k] - 0.5 * p[NSIMP][k];
+            // lane 0 reflection, 1 expansion, 2 contraction, 4..7 the points 1..4 shrunk
+            const double w = o == 4 ? p[1][k] : o == 5 ? p[2][k] : o == 6 ? p[3][k] : p[4][k];
+            q[k] = o == 0 ? t[k] : o == 1 ? se[k] : o == 2 ? sc[k] : 0.5 * (w + p[0][k]);
+        }
+        double x = chi2max;
+        if (act && o != 3 && (o > 3 || !out_of_box(q))) x = chi2_string(ph, q);
+        const double chi2 = __shfl(x, 0, OCT), chi2e = __shfl(x, 1, OCT), chi2c = __shfl(x, 2, OCT);
+        double x2[NSIMP];
+#pragma unroll
+        for (int a = 0; a < NSIMP; a++) x2[a] = __shfl(x, 4 + a, OCT);
+        if (act) {
+            if (chi2 < c2[NSIMP]) {
+                if (chi2 <= chi2e) { c2[NSIMP] = chi2; copy4(p[NSIMP], t); }
+                else { c2[NSIMP] = chi2e; copy4(p[NSIMP], se); }
+            } else if (chi2c <= c2[NSIMP]) {
+                c2[NSIMP] = chi2c;
+                copy4(p[NSIMP], sc);
+            } else {
+#pragma unroll
+                for (int i0 = 1; i0 <= NSIMP; i0++) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) p[i0][k] = 0.5 * (p[i0][k] + p[0][k]);
+                    c2[i0] = x2[i0 - 1];
+                }
+            }
+            sort_simplex(p, c2);
+        }
     }
 }
 
@@ -520,40 +712,78 @@ __device__ __forceinline__ void finish_string(const typename V2<T>::type* __rest
     o[10] = vel[2];
 }
 
-// Searches parked by stage one: slot j holds string pend[j] and, at state + 26 j, its simplex
-// points (20), their chi2 (5) and the iterations done.
+// The searches between the kernels: at state + 26 s, string s's simplex points (20), their chi2 (5) and the
+// iterations done.
 
-// Stage one: random starts and the first `split` simplex iterations of string s = one thread.
+// Stage one: the random starts of string s = one octet, into its state.
 template <typename T, bool COMP>
-__global__ void __launch_bounds__(STRING_NT) string_fit_kernel(int N, const typename V2<T>::type* __restrict__ phi,
-                                                               const short2* __restrict__ cphi,
-                                                               const typename V2<T>::type* __restrict__ pi,
-                                                               const short2* __restrict__ cpi,
-                                                               const int32_t* __restrict__ cells, int64_t ns,
-                                                               Draws dr, double dspa, int split,
-                                                               double* __restrict__ rec, int* __restrict__ npend,
-                                                               int64_t* __restrict__ pend, double* __restrict__ state)
+__global__ void __launch_bounds__(STRING_NT, 3) string_starts_kernel(int N, const typename V2<T>::type* __restrict__ phi,
+                                                                  const short2* __restrict__ cphi,
+                                                                  const int32_t* __restrict__ cells, int64_t ns, Draws dr,
+                                                                  double* __restrict__ state)
+{
+#pragma clang fp contract(off)
+    __shared__ uint16_t queue[64 / OCT][START_Q];
+    const int64_t s = blockIdx.x * (int64_t)(STRING_NT / OCT) + threadIdx.x / OCT;
+    const bool valid = s < ns;
+    // an octet past the last string repeats the first one's cell and only takes part in the votes
+    const Phases ph = corner_phases<T, COMP>(phi, cphi, string_cell(N, cells, valid ? s : 0));
+    double p[NSIMP + 1][4], c2[NSIMP + 1];
+    fit_starts(ph, dr, s, valid, queue, p, c2);
+    if (!valid) return;
+    double* st = state + s * STRING_STATE;
+    const int o = threadIdx.x & (OCT - 1);
+#pragma unroll
+    for (int a = 0; a <= NSIMP; a++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (((4 * a + k) & (OCT - 1)) == o) st[4 * a + k] = p[a][k];
+        if (((20 + a) & (OCT - 1)) == o) st[20 + a] = c2[a];
+    }
+    if ((25 & (OCT - 1)) == o) st[25] = 0;
+}
+
+// Stages two and three: the simplex iterations of the n strings (list null: all of them; else *count strings of the
+// list) up to itmax, one string per lane.  A string still searching goes back to its state and onto
+// pend; the others get their records.  Two waves a SIMD (206 VGPRs); in 168 VGPRs it spills 41 of them
+// and is no faster (512^3, both kernels: 37 ms either way).
+static_assert(STRING_NT == 64, "string fit blocks are one wave (see ShrinkLds)");
+template <typename T, bool COMP>
+__global__ void __launch_bounds__(STRING_NT, 2) string_fit_kernel(
+    int N, const typename V2<T>::type* __restrict__ phi, const short2* __restrict__ cphi,
+    const typename V2<T>::type* __restrict__ pi, const short2* __restrict__ cpi, const int32_t* __restrict__ cells,
+    double dspa, double* __restrict__ rec, int64_t n, const int* __restrict__ count, const int64_t* __restrict__ list,
+    int itmax, int* __restrict__ npend, int64_t* __restrict__ pend, double* __restrict__ state)
 {
 #pragma clang fp contract(off)
     __shared__ ShrinkLds lds;
-    const int64_t s = blockIdx.x * (int64_t)STRING_NT + threadIdx.x;
+    if (list) n = *count;
+    if (blockIdx.x * (int64_t)STRING_NT >= n) return;  // the whole wave has no search
+    const int64_t j = blockIdx.x * (int64_t)STRING_NT + threadIdx.x;
     // lanes past the last string stay for the wave's shared shrink evaluations
-    const bool valid = s < ns;
-    const StringCell sc = string_cell(N, cells, valid ? s : 0);
-    Phases ph;
+    const bool valid = j < n;
     double p[NSIMP + 1][4], c2[NSIMP + 1];
     int it = 0;
+    Phases ph;
     if (valid) {
-        ph = corner_phases<T, COMP>(phi, cphi, sc);
-        fit_starts(ph, dr, s, p, c2);
+        const int64_t s = list ? list[j] : j;
+        const double* st = state + s * STRING_STATE;
+#pragma unroll
+        for (int a = 0; a <= NSIMP; a++) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) p[a][k] = st[4 * a + k];
+            c2[a] = st[20 + a];
+        }
+        it = (int)st[25];
+        ph = corner_phases<T, COMP>(phi, cphi, string_cell(N, cells, s));
     }
-    fit_simplex(ph, p, c2, it, split < MAXIT ? split : MAXIT, valid, lds);
+    fit_simplex(ph, p, c2, it, itmax, valid, lds);
     if (!valid) return;
+    const int64_t s = list ? list[j] : j;  // read again rather than kept live through the search
     if (c2[0] > STR_TOL && it < MAXIT) {
-        // still searching: park it for stage two
-        const int j = atomicAdd(npend, 1);
-        pend[j] = s;
-        double* st = state + (int64_t)j * STRING_STATE;
+        // still searching: back to its state, for the next stage
+        pend[atomicAdd(npend, 1)] = s;
+        double* st = state + s * STRING_STATE;
 #pragma unroll
         for (int a = 0; a <= NSIMP; a++) {
 #pragma unroll
@@ -565,48 +795,38 @@ __global__ void __launch_bounds__(STRING_NT) string_fit_kernel(int N, const type
     }
     double pos[3], dir[3], gof, sl;
     fit_result(p[0], c2[0], pos, dir, gof, sl);
-    finish_string<T, COMP>(phi, cphi, pi, cpi, sc, pos, dir, gof, sl, dspa, rec, s);
+    finish_string<T, COMP>(phi, cphi, pi, cpi, string_cell(N, cells, s), pos, dir, gof, sl, dspa, rec, s);
 }
 
-// Stage two: the parked searches, one per thread, continued to the end.
-constexpr int STRING_NT2 = 64;
-static_assert(STRING_NT2 == 64, "string fit blocks are one wave (see ShrinkLds)");
+// The simplex of every string from its starts, one octet per string, where the strings are few: a search of
+// 1000 iterations is one chain of chi2 whatever the number of searches, 9.6 ms for lanes and 3 ms
+// for octets, and up to OCT_MAX strings the octets' waves are at most two a SIMD.  From there the lanes'
+// three and a half rounds for 64 strings beat the octets' one for eight.
+constexpr int64_t OCT_MAX = 16384;
 template <typename T, bool COMP>
-__global__ void __launch_bounds__(STRING_NT2, 3) string_fit_rest_kernel(
+__global__ void __launch_bounds__(STRING_NT, 2) string_fit_oct_kernel(
     int N, const typename V2<T>::type* __restrict__ phi, const short2* __restrict__ cphi,
     const typename V2<T>::type* __restrict__ pi, const short2* __restrict__ cpi, const int32_t* __restrict__ cells,
-    double dspa, double* __restrict__ rec, const int* __restrict__ npend, const int64_t* __restrict__ pend,
-    const double* __restrict__ state)
+    double dspa, double* __restrict__ rec, int64_t ns, const double* __restrict__ state)
 {
 #pragma clang fp contract(off)
-    __shared__ ShrinkLds lds;
-    const int np = *npend;
-    if (blockIdx.x * STRING_NT2 >= (unsigned)np) return;  // the whole wave has no search
-    const int j = blockIdx.x * STRING_NT2 + threadIdx.x;
-    const bool valid = j < np;
+    const int64_t s = blockIdx.x * (int64_t)(STRING_NT / OCT) + threadIdx.x / OCT;
+    const bool valid = s < ns;
+    const int64_t r = valid ? s : 0;
+    const Phases ph = corner_phases<T, COMP>(phi, cphi, string_cell(N, cells, r));
     double p[NSIMP + 1][4], c2[NSIMP + 1];
-    int it = 0;
-    Phases ph;
-    StringCell sc{N, 0, 0, 0};
-    int64_t s = 0;
-    if (valid) {
-        s = pend[j];
-        const double* st = state + (int64_t)j * STRING_STATE;
+    const double* st = state + r * STRING_STATE;
 #pragma unroll
-        for (int a = 0; a <= NSIMP; a++) {
+    for (int a = 0; a <= NSIMP; a++) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) p[a][k] = st[4 * a + k];
-            c2[a] = st[20 + a];
-        }
-        it = (int)st[25];
-        sc = string_cell(N, cells, s);
-        ph = corner_phases<T, COMP>(phi, cphi, sc);
+        for (int k = 0; k < 4; k++) p[a][k] = st[4 * a + k];
+        c2[a] = st[20 + a];
     }
-    fit_simplex(ph, p, c2, it, MAXIT, valid, lds);
-    if (!valid) return;
+    fit_simplex_oct(ph, p, c2, valid);
+    if (!valid || (threadIdx.x & (OCT - 1)) != 0) return;
     double pos[3], dir[3], gof, sl;
     fit_result(p[0], c2[0], pos, dir, gof, sl);
-    finish_string<T, COMP>(phi, cphi, pi, cpi, sc, pos, dir, gof, sl, dspa, rec, s);
+    finish_string<T, COMP>(phi, cphi, pi, cpi, string_cell(N, cells, s), pos, dir, gof, sl, dspa, rec, s);
 }
 
 // velocity_string_YY (defects_3d.f90:824-982, the reference's VEL = 1 build) for string cell s,
@@ -793,16 +1013,25 @@ void launch_string_fit(hipStream_t s, int N, const void* phi, const void* cphi, 
     if (ns > INT32_MAX) throw Error(AXG_EINVAL, "string fits: more than 2^31 - 1 string cells");
     const int64_t nblk = (ns + STRING_NT - 1) / STRING_NT;
     AXG_HIP(hipMemsetAsync(npend, 0, sizeof(int), s));
-    hipLaunchKernelGGL((string_fit_kernel<T, COMP>), dim3((unsigned)nblk), dim3(STRING_NT), 0, s, N, (const T2*)phi,
-                       (const short2*)cphi, (const T2*)pi, (const short2*)cpi, cells, ns, dr, dspa, split, rec,
-                       npend, pend, state);
+    hipLaunchKernelGGL((string_starts_kernel<T, COMP>), dim3((unsigned)((ns * OCT + STRING_NT - 1) / STRING_NT)),
+                       dim3(STRING_NT), 0, s, N, (const T2*)phi, (const short2*)cphi, cells, ns, dr, state);
     AXG_HIP(hipGetLastError());
-    // as many threads as strings; waves past the parked count return at once
-    hipLaunchKernelGGL((string_fit_rest_kernel<T, COMP>), dim3((unsigned)((ns + STRING_NT2 - 1) / STRING_NT2)),
-                       dim3(STRING_NT2), 0, s, N, (const T2*)phi, (const short2*)cphi, (const T2*)pi,
-                       (const short2*)cpi, cells, dspa, rec, (const int*)npend, (const int64_t*)pend,
-                       (const double*)state);
-    AXG_HIP(hipGetLastError());
+    auto fit = [&](const int64_t* list, int itmax) {
+        hipLaunchKernelGGL((string_fit_kernel<T, COMP>), dim3((unsigned)nblk), dim3(STRING_NT), 0, s, N, (const T2*)phi,
+                           (const short2*)cphi, (const T2*)pi, (const short2*)cpi, cells, dspa, rec, ns, (const int*)npend,
+                           list, itmax, npend, pend, state);
+        AXG_HIP(hipGetLastError());
+    };
+    if (ns <= OCT_MAX) {
+        hipLaunchKernelGGL((string_fit_oct_kernel<T, COMP>), dim3((unsigned)((ns * OCT + STRING_NT - 1) / STRING_NT)),
+                           dim3(STRING_NT), 0, s, N, (const T2*)phi, (const short2*)cphi, (const T2*)pi, (const short2*)cpi,
+                           cells, dspa, rec, ns, (const double*)state);
+        AXG_HIP(hipGetLastError());
+    } else {
+        fit(nullptr, split < MAXIT ? split : MAXIT);
+        // as many threads as strings; waves past the parked count return at once
+        fit(pend, MAXIT);
+    }
     if (vel_yy) {
         hipLaunchKernelGGL((string_vel_yy_kernel<T, COMP>), dim3((unsigned)nblk), dim3(STRING_NT), 0, s, N,
                            (const T2*)phi, (const short2*)cphi, (const T2*)pi, (const short2*)cpi, cells, ns, dspa, rec);
