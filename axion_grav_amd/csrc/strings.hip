@@ -505,12 +505,22 @@ __device__ __forceinline__ void fit_simplex(const Phases& ph, double (&p)[NSIMP 
                     c2[NSIMP] = chi2s;
                     copy4(p[NSIMP], sv);
                 } else {
-                    // shrink towards the best point
+                    // shrink towards the best point; a search that has collapsed to its last bits
+                    // (four in five of the shrinks after the 200th iteration) gets points whose
+                    // chi2 it has: the same point again, or the best point
 #pragma unroll
-                    for (int i0 = 1; i0 <= NSIMP; i0++)
+                    for (int i0 = 1; i0 <= NSIMP; i0++) {
+                        bool same = true, best = true;
 #pragma unroll
-                        for (int k = 0; k < 4; k++) p[i0][k] = 0.5 * (p[i0][k] + p[0][k]);
-                    shr = true;
+                        for (int k = 0; k < 4; k++) {
+                            const double q = 0.5 * (p[i0][k] + p[0][k]);
+                            same = same && q == p[i0][k];
+                            best = best && q == p[0][k];
+                            p[i0][k] = q;
+                        }
+                        if (best) c2[i0] = c2[0];
+                        shr = shr || !(same || best);
+                    }
                 }
             }
         }
@@ -746,7 +756,7 @@ __global__ void __launch_bounds__(STRING_NT, 3) string_starts_kernel(int N, cons
 // Stages two and three: the simplex iterations of the n strings (list null: all of them; else *count strings of the
 // list) up to itmax, one string per lane.  A string still searching goes back to its state and onto
 // pend; the others get their records.  Two waves a SIMD (206 VGPRs); in 168 VGPRs it spills 41 of them
-// and is no faster (512^3, both kernels: 37 ms either way).
+// and is no faster (512^3, both kernels: 33 ms).
 static_assert(STRING_NT == 64, "string fit blocks are one wave (see ShrinkLds)");
 template <typename T, bool COMP>
 __global__ void __launch_bounds__(STRING_NT, 2) string_fit_kernel(
@@ -799,7 +809,7 @@ __global__ void __launch_bounds__(STRING_NT, 2) string_fit_kernel(
 }
 
 // The simplex of every string from its starts, one octet per string, where the strings are few: a search of
-// 1000 iterations is one chain of chi2 whatever the number of searches, 9.6 ms for lanes and 3 ms
+// 1000 iterations is one chain of chi2 whatever the number of searches, 8.9 ms for lanes and 4.7 ms
 // for octets, and up to OCT_MAX strings the octets' waves are at most two a SIMD.  From there the lanes'
 // three and a half rounds for 64 strings beat the octets' one for eight.
 constexpr int64_t OCT_MAX = 16384;
