@@ -35,7 +35,12 @@ constexpr int WALL_GRID = 20;
 struct WallGrid {
     double smu[WALL_GRID];         // sqrt(1 - mu^2) of mu index imu - 1
     double cs[WALL_GRID][2];       // cos, sin of phi index iphi - 1
+    double cs2[WALL_GRID][2];      // cos^2 - 1/2, cos sin: cos 2phi / 2, sin 2phi / 2
 };
+
+// Above twice the difference of the two forms of chi2 (each a sum of some 60 products of at most 12 * 0.75 = 9 in
+// FP64: 60 * 9 * 2^-53 = 6e-14 each).
+constexpr double WALL_EPS = 1e-11;
 
 __device__ __forceinline__ double grid_mu(int imu) { return (-20 + 2 * imu - 1.0) / 20; }
 __device__ __forceinline__ double grid_phi(int iphi) { return PI_T * (2 * iphi - 1.0 - 20) / 20; }
@@ -66,32 +71,92 @@ __device__ int position_wall(const double ph[8], const WallGrid& G, double pos[3
     for (int e = 0; e < 12; e++) m += ok[e] ? 1 : 0;
     if (m < 3) return m;
 
-    double chi2min = 6.0, mut = 0, wt = 0;
-    int bphi = 0;  // phi index of the best direction (0: none below chi2 = 6)
-    for (int imu = 1; imu <= WALL_GRID; imu++) {
-        const double mu = grid_mu(imu), smu = G.smu[imu - 1];
-        for (int iphi = 1; iphi <= WALL_GRID; iphi++) {
-            const double d0 = smu * G.cs[iphi - 1][0], d1 = smu * G.cs[iphi - 1][1], d2 = mu;
-            double w = 0, chi2 = 0;
+    // The search takes the first direction of least chi2 = sum d^2 - m w^2, w = max(0, sum d) / m, d = point .
+    // direction: 400 directions of up to 12 points.  sum d^2 is a quadratic form of the direction and sum d
+    // a linear one, so for one mu both are trigonometric polynomials of phi, ten multiply-adds a
+    // direction.  That form is rounded in another order, by less than WALL_EPS, so it is only used to find
+    // the directions that can be the least; their chi2 are then taken point by point, in the
+    // search's own order: one direction, unless the second best is within WALL_EPS of the best.  Records are
+    // the same bit for bit.  512^3, 7.1 M cells: 13.9 -> 3.5 ms; 256^3 2.2 -> 0.55 ms.  (The loop over
+    // mu kept rolled, 128 VGPRs: unrolled it took 256, 5 ms.)
+    double qxx = 0, qyy = 0, qzz = 0, qxy = 0, qxz = 0, qyz = 0, sx = 0, sy = 0, sz = 0;
 #pragma unroll
-            for (int e = 0; e < 12; e++) {
-                if (!ok[e]) continue;
-                double px, py, pz;
-                edge_point(e, t[e], px, py, pz);
-                const double d = px * d0 + py * d1 + pz * d2;
-                w = w + d;
-                chi2 = chi2 + d * d;
-            }
-            if (w < 0) w = 0;
-            else w = w / m;
-            chi2 = chi2 - m * w * w;
-            if (chi2 < chi2min) {
-                chi2min = chi2;
-                mut = mu;
-                bphi = iphi;
-                wt = w;
+    for (int e = 0; e < 12; e++) {
+        if (!ok[e]) continue;
+        double px, py, pz;
+        edge_point(e, t[e], px, py, pz);
+        qxx += px * px;
+        qyy += py * py;
+        qzz += pz * pz;
+        qxy += px * py;
+        qxz += px * pz;
+        qyz += py * pz;
+        sx += px;
+        sy += py;
+        sz += pz;
+    }
+    const double im = 1.0 / m;
+    auto estimates = [&](auto&& use) {
+#pragma unroll 1
+        for (int imu = 1; imu <= WALL_GRID; imu++) {
+            const double mu = grid_mu(imu), smu = G.smu[imu - 1], s2 = smu * smu;
+            // sum d^2 = c0 + c1 cos phi + c2 sin phi + c3 cos 2phi / 2 + c4 sin 2phi / 2, sum d = l0 + l1 cos + l2 sin
+            const double c0 = 0.5 * s2 * (qxx + qyy) + mu * mu * qzz, c1 = 2 * smu * mu * qxz, c2 = 2 * smu * mu * qyz;
+            const double c3 = s2 * (qxx - qyy), c4 = 2 * s2 * qxy;
+            const double l0 = mu * sz, l1 = smu * sx, l2 = smu * sy;
+#pragma unroll 4
+            for (int iphi = 1; iphi <= WALL_GRID; iphi++) {
+                const double co = G.cs[iphi - 1][0], si = G.cs[iphi - 1][1];
+                const double co2 = G.cs2[iphi - 1][0], si2 = G.cs2[iphi - 1][1];
+                double q = fma(c1, co, c0);
+                q = fma(c2, si, q);
+                q = fma(c3, co2, q);
+                q = fma(c4, si2, q);
+                const double l = fmax(fma(l2, si, fma(l1, co, l0)), 0.0);
+                use(imu, iphi, fma(-(l * im), l, q));
             }
         }
+    };
+    double best = 1e300, second = 1e300;
+    int ibest = 1, jbest = 1;
+    estimates([&](int imu, int iphi, double c) {
+        const bool less = c < best;
+        second = less ? best : fmin(second, c);
+        best = less ? c : best;
+        ibest = less ? imu : ibest;
+        jbest = less ? iphi : jbest;
+    });
+    double chi2min = 6.0, mut = 0, wt = 0;
+    int bphi = 0;  // phi index of the best direction (0: none below chi2 = 6)
+    auto test = [&](int imu, int iphi) {
+        const double mu = grid_mu(imu), smu = G.smu[imu - 1];
+        const double d0 = smu * G.cs[iphi - 1][0], d1 = smu * G.cs[iphi - 1][1], d2 = mu;
+        double w = 0, chi2 = 0;
+#pragma unroll
+        for (int e = 0; e < 12; e++) {
+            if (!ok[e]) continue;
+            double px, py, pz;
+            edge_point(e, t[e], px, py, pz);
+            const double d = px * d0 + py * d1 + pz * d2;
+            w = w + d;
+            chi2 = chi2 + d * d;
+        }
+        if (w < 0) w = 0;
+        else w = w / m;
+        chi2 = chi2 - m * w * w;
+        if (chi2 < chi2min) {
+            chi2min = chi2;
+            mut = mu;
+            bphi = iphi;
+            wt = w;
+        }
+    };
+    if (second > best + WALL_EPS) {
+        test(ibest, jbest);
+    } else {
+        estimates([&](int imu, int iphi, double c) {
+            if (c <= best + WALL_EPS) test(imu, iphi);
+        });
     }
     const double phit = bphi > 0 ? grid_phi(bphi) : 0.0;
     double dr[3] = {sqrt(1 - mut * mut) * cos(phit), sqrt(1 - mut * mut) * sin(phit), mut};
@@ -169,7 +234,7 @@ __device__ int position_wall(const double ph[8], const WallGrid& G, double pos[3
 }
 
 template <typename T, bool COMP>
-__global__ void __launch_bounds__(WALL_NT) wall_fit_kernel(int N, const typename V2<T>::type* __restrict__ phi,
+__global__ void __launch_bounds__(WALL_NT, 4) wall_fit_kernel(int N, const typename V2<T>::type* __restrict__ phi,
                                                            const short2* __restrict__ cphi,
                                                            const int32_t* __restrict__ cells, int64_t nw,
                                                            double* __restrict__ rec, double* __restrict__ partial)
@@ -183,6 +248,8 @@ __global__ void __launch_bounds__(WALL_NT) wall_fit_kernel(int N, const typename
         grid.smu[threadIdx.x] = sqrt(1 - mu * mu);
         grid.cs[threadIdx.x][0] = cos(phi);
         grid.cs[threadIdx.x][1] = sin(phi);
+        grid.cs2[threadIdx.x][0] = cos(phi) * cos(phi) - 0.5;
+        grid.cs2[threadIdx.x][1] = cos(phi) * sin(phi);
     }
     __syncthreads();
     const int64_t s = blockIdx.x * (int64_t)WALL_NT + threadIdx.x;
