@@ -268,6 +268,7 @@ struct axg_handle {
             gs->release();
             delete gs;
             gs = nullptr;
+            staging_release(p.device);
         }
         for (auto e : ev) (void)hipEventDestroy(e);
         ev.clear();
@@ -575,6 +576,7 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         h->release();
         return AXG_ENOMEM;
     }
+    staging_retain(p.device);
     *out = h.release();
     return AXG_OK;
 }
@@ -584,8 +586,10 @@ extern "C" int axg_destroy(axg_handle* h)
     if (!h) return AXG_EINVAL;
     (void)hipSetDevice(h->p.device);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
+    const int device = h->p.device;
     h->release();
     delete h;
+    staging_release(device);
     return AXG_OK;
 }
 
@@ -617,11 +621,11 @@ extern "C" int axg_set_fields(axg_handle* h, const double* phi, const double* pi
         require(nsite == h->n3, "nsite must be ngrid^3");
         size_t bytes = (size_t)h->n3 * 16;
         if (phi) {
-            AXG_HIP(hipMemcpyAsync(h->work, phi, bytes, hipMemcpyHostToDevice, h->stream));
+            copy_to_device(h->p.device, h->stream, h->work, phi, bytes);
             store_from_work(h, h->phi[h->cur], h->cphi[h->cur]);
         }
         if (pi) {
-            AXG_HIP(hipMemcpyAsync(h->work, pi, bytes, hipMemcpyHostToDevice, h->stream));
+            copy_to_device(h->p.device, h->stream, h->work, pi, bytes);
             store_from_work(h, h->pi, h->cpi);
         }
         h->have_flags = false;
@@ -641,13 +645,11 @@ extern "C" int axg_get_fields(axg_handle* h, double* phi, double* pi, int64_t ns
         size_t bytes = (size_t)h->n3 * 16;
         if (phi) {
             load_to_work(h, h->phi[h->cur], h->cphi[h->cur]);
-            AXG_HIP(hipMemcpyAsync(phi, h->work, bytes, hipMemcpyDeviceToHost, h->stream));
-            AXG_HIP(hipStreamSynchronize(h->stream));
+            copy_to_host(h->p.device, h->stream, phi, h->work, bytes);
         }
         if (pi) {
             load_to_work(h, h->pi, h->cpi);
-            AXG_HIP(hipMemcpyAsync(pi, h->work, bytes, hipMemcpyDeviceToHost, h->stream));
-            AXG_HIP(hipStreamSynchronize(h->stream));
+            copy_to_host(h->p.device, h->stream, pi, h->work, bytes);
         }
     });
 }
@@ -671,8 +673,7 @@ extern "C" int axg_get_gw_state(axg_handle* h, double* A, int64_t count)
         for (int m = 0; m < 4; m++) {
             if (h->fp32) launch_gw_pack<float>(h->stream, N, h->L, h->A, m, h->work, +1);
             else launch_gw_pack<double>(h->stream, N, h->L, h->A, m, h->work, +1);
-            AXG_HIP(hipMemcpyAsync(A + 2 * per * m, h->work, per * 16, hipMemcpyDeviceToHost, h->stream));
-            AXG_HIP(hipStreamSynchronize(h->stream));
+            copy_to_host(h->p.device, h->stream, A + 2 * per * m, h->work, per * 16);
         }
     });
 }
@@ -686,7 +687,7 @@ extern "C" int axg_set_gw_state(axg_handle* h, const double* A, int64_t count)
         require(A && count == (int64_t)4 * N * N * h->nh, "count must be 4*N*N*(N/2+1)");
         const size_t per = (size_t)N * N * h->nh;
         for (int m = 0; m < 4; m++) {
-            AXG_HIP(hipMemcpyAsync(h->work, A + 2 * per * m, per * 16, hipMemcpyHostToDevice, h->stream));
+            copy_to_device(h->p.device, h->stream, h->work, A + 2 * per * m, per * 16);
             if (h->fp32) launch_gw_pack<float>(h->stream, N, h->L, h->A, m, h->work, -1);
             else launch_gw_pack<double>(h->stream, N, h->L, h->A, m, h->work, -1);
             AXG_HIP(hipStreamSynchronize(h->stream));
@@ -1168,9 +1169,7 @@ extern "C" int axg_get_plaquettes(axg_handle* h, int32_t* rec, int64_t cap, int6
         }
         const int64_t nblk = (h->n3 + PLAQ_BLOCK - 1) / PLAQ_BLOCK;
         launch_plaquette_compact(h->stream, h->N, h->plaq_code, h->plaq_cnt + 16 * nblk, h->plaq_rec);
-        AXG_HIP(hipMemcpyAsync(rec, h->plaq_rec, (size_t)5 * h->nplaq * sizeof(int32_t), hipMemcpyDeviceToHost,
-                               h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
+        copy_to_host(h->p.device, h->stream, rec, h->plaq_rec, (size_t)5 * h->nplaq * sizeof(int32_t));
     });
 }
 
@@ -1186,8 +1185,7 @@ extern "C" int axg_get_mask(axg_handle* h, int32_t* ixyz, int64_t cap, int64_t* 
         int64_t* offs = h->blk + 3 * nblk;
         int32_t* dm = (int32_t*)h->work;  // 3*nmask ints fit in the N^3 x 16-byte work array
         launch_cell_compact(h->stream, h->N, h->flags, 4, offs, dm, 1, nblk);
-        AXG_HIP(hipMemcpyAsync(ixyz, dm, (size_t)3 * h->nmask * sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
+        copy_to_host(h->p.device, h->stream, ixyz, dm, (size_t)3 * h->nmask * sizeof(int32_t));
     });
 }
 
@@ -1438,9 +1436,7 @@ extern "C" int axg_get_walls(axg_handle* h, double* rec, int64_t cap, int64_t* c
         *count = h->nwall_rec;
         if (h->nwall_rec == 0 || rec == nullptr || cap == 0) return;  // size query
         require(cap >= h->nwall_rec, "wall buffer too small");
-        AXG_HIP(hipMemcpyAsync(rec, h->wall_rec, (size_t)8 * h->nwall_rec * sizeof(double), hipMemcpyDeviceToHost,
-                               h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
+        copy_to_host(h->p.device, h->stream, rec, h->wall_rec, (size_t)8 * h->nwall_rec * sizeof(double));
     });
 }
 
@@ -1452,9 +1448,7 @@ extern "C" int axg_get_strings(axg_handle* h, double* rec, int64_t cap, int64_t*
         *count = h->nstr_rec;
         if (h->nstr_rec == 0 || rec == nullptr || cap == 0) return;  // size query
         require(cap >= h->nstr_rec, "string buffer too small");
-        AXG_HIP(hipMemcpyAsync(rec, h->str_rec, (size_t)11 * h->nstr_rec * sizeof(double), hipMemcpyDeviceToHost,
-                               h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
+        copy_to_host(h->p.device, h->stream, rec, h->str_rec, (size_t)11 * h->nstr_rec * sizeof(double));
     });
 }
 
@@ -1463,8 +1457,7 @@ extern "C" int axg_get_flags(axg_handle* h, int8_t* flags, int64_t nsite)
     return guarded(h, [&] {
         require(h->have_flags, "call axg_defects first");
         require(flags && nsite == h->n3, "nsite must be ngrid^3");
-        AXG_HIP(hipMemcpyAsync(flags, h->flags, h->n3, hipMemcpyDeviceToHost, h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
+        copy_to_host(h->p.device, h->stream, flags, h->flags, h->n3);
     });
 }
 
@@ -2256,15 +2249,15 @@ extern "C" int axg_get_adjoint(axg_handle* h, double* phibar, double* pibar, int
     return guarded(h, [&] {
         require(h->have_adj, "call axg_gradient first");
         require(nsite == h->n3, "nsite must be N^3");
-        if (phibar)
-            AXG_HIP(hipMemcpyAsync(phibar, h->adj, (size_t)h->n3 * sizeof(double2), hipMemcpyDeviceToHost, h->stream));
-        if (pibar)
-            AXG_HIP(hipMemcpyAsync(pibar, h->adj_pibar, (size_t)h->n3 * sizeof(double2), hipMemcpyDeviceToHost,
-                                   h->stream));
-        AXG_HIP(hipStreamSynchronize(h->stream));
-        for (int64_t i = 0; i < 2 * h->n3; i++) {
-            if (phibar) phibar[i] *= h->adj_scale;
-            if (pibar) pibar[i] *= h->adj_scale;
+        // scaled on the device, through the work array
+        const size_t bytes = (size_t)h->n3 * sizeof(double2);
+        if (phibar) {
+            launch_scaled_copy(h->stream, h->n3, h->adj, h->adj_scale, h->work);
+            copy_to_host(h->p.device, h->stream, phibar, h->work, bytes);
+        }
+        if (pibar) {
+            launch_scaled_copy(h->stream, h->n3, h->adj_pibar, h->adj_scale, h->work);
+            copy_to_host(h->p.device, h->stream, pibar, h->work, bytes);
         }
     });
 }
