@@ -320,12 +320,22 @@ __device__ __forceinline__ void p2_exchange_if(bool active, typename V2<T>::type
     __syncthreads();
 }
 
+// A workgroup barrier for LDS traffic only: this wave's LDS operations complete, then s_barrier.
+// __syncthreads() also waits (vmcnt 0) for every direct global-to-LDS copy in flight, since such a
+// copy writes LDS; a transform that runs while its block copies its next input into another LDS
+// tile synchronises with this barrier instead (fft_p2_rb), which leaves the copies in flight.
+__device__ __forceinline__ void lds_sync()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // The radix-3 step of N = 3 * 2^L after the last register stage (span PW = N/3).  Its
 // butterfly j < PW maps y[j + r PW] to X[j + r' PW] = sum_r y[j + r PW] w^(r j) w3^(r r')
 // with w = exp(SIGN 2 pi i/N), w3 = w^PW, i.e. X[n] = sum_r y[(n mod PW) + r PW] w^(r n).  The
 // thread's outputs n = j0 + e TPT (TPT = N/8) need w^n = w^j0 exp(SIGN 2 pi i e/8) and
 // w^(2n) = w^(2 j0) exp(SIGN 2 pi i 2e/8), so two table twiddles serve all eight.
-template <typename T, int N, int SIGN, typename TW>
+// RB: lds_sync barriers.
+template <typename T, int N, int SIGN, bool RB = false, typename TW>
 __device__ __forceinline__ void p3_finish(bool active, typename V2<T>::type (&v)[8], int j0, typename V2<T>::type* s,
                                           int es, int off, const TW& tws)
 {
@@ -342,7 +352,8 @@ __device__ __forceinline__ void p3_finish(bool active, typename V2<T>::type (&v)
             for (int r = 0; r < R; r++) s[(base + r * Ns) * es + off] = v[m + r * M];
         }
     }
-    __syncthreads();
+    if constexpr (RB) lds_sync();
+    else __syncthreads();
     if (active) {
         const T2 a = p3_tw(tws, 0), b = p3_tw(tws, 1);
         [&]<int... E>(std::integer_sequence<int, E...>) {
@@ -356,7 +367,8 @@ __device__ __forceinline__ void p3_finish(bool active, typename V2<T>::type (&v)
                 ...);
         }(std::make_integer_sequence<int, 8>{});
     }
-    __syncthreads();
+    if constexpr (RB) lds_sync();
+    else __syncthreads();
 }
 
 // One radix-9 pass of span Ns on a transform in LDS (element n at s[n*es + off]): thread slot j < N/9
@@ -495,15 +507,6 @@ __device__ __forceinline__ void fft_p2(typename V2<T>::type (&v)[8], int j0, typ
     }
 }
 
-// A workgroup barrier for LDS traffic only: this wave's LDS operations complete, then s_barrier.
-// __syncthreads() also waits (vmcnt 0) for every direct global-to-LDS copy in flight, since such a
-// copy writes LDS; a transform that runs while its block copies its next input into another LDS
-// tile synchronises with this barrier instead (fft_p2_rb), which leaves the copies in flight.
-__device__ __forceinline__ void lds_sync()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 template <typename T, int N, int S>
 __device__ __forceinline__ void p2_exchange_rb(typename V2<T>::type (&v)[8], int j0, typename V2<T>::type* s, int es, int off)
 {
@@ -522,7 +525,7 @@ __device__ __forceinline__ void p2_exchange_rb(typename V2<T>::type (&v)[8], int
     lds_sync();
 }
 
-// fft_p2 with lds_sync barriers (2^k sizes).
+// fft_p2 with lds_sync barriers (2^k and 3 * 2^k sizes).
 template <typename T, int N, int SIGN, int S = 0, typename TW>
 __device__ __forceinline__ void fft_p2_rb(typename V2<T>::type (&v)[8], int j0, typename V2<T>::type* s, int es, int off,
                                           const TW& tws)
@@ -530,8 +533,17 @@ __device__ __forceinline__ void fft_p2_rb(typename V2<T>::type (&v)[8], int j0, 
     if constexpr (S < P2<N>::NST) {
         p2_stage<T, N, S, SIGN>(v, tws);
         if constexpr (S + 1 < P2<N>::NST) p2_exchange_rb<T, N, S>(v, j0, s, es, off);
+        else if constexpr (P2<N>::R3) p3_finish<T, N, SIGN, true>(true, v, j0, s, es, off, tws);
         fft_p2_rb<T, N, SIGN, S + 1>(v, j0, s, es, off, tws);
     }
+}
+
+// Keeps a transform's last arithmetic where it is: used only behind a branch or after another transform, it
+// would be moved down there, and its LDS inputs (three values for one output in p3_finish) held until then.
+template <typename T2> __device__ __forceinline__ void p2_pin(T2 (&v)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 8; e++) asm volatile("" : "+v"(v[e].x), "+v"(v[e].y));
 }
 
 // Two transforms per thread, the LDS tile's columns off0 and off1, through the same stages: the

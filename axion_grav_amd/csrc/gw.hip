@@ -240,6 +240,99 @@ __global__ void __launch_bounds__((TX / 2) * (N / 8)) gw_ypass_p2w_kernel(const 
     }
 }
 
+// The y pass of gw_ypass_p2w_kernel for the FP32 sizes whose tile leaves a CU one block, so that nothing
+// runs there while the block's loads are on their way (and two planes' values in registers spill).  A
+// block takes NP planes in turn; the next plane's tile is copied into LDS by direct
+// global-to-LDS loads while the current one is transformed, one column of a thread's pair after the other
+// through half a tile (lds_sync barriers and LDS twiddles, as in the z pass, so that nothing waits
+// for the copies).  Two planes' outputs for one (ky, kx) are adjacent tile rows: the first one's are
+// held and both stored back to back.  768^3 FP32C: 7.58 -> 4.51 ms (5.1 TB/s of its 23.1 GB; the
+// two-plane two-column kernel 6.8 with its spills taken out); at 1024 the tile and a half do not fit, at 576 and
+// 648 the radix-9 passes wait for the copies.  NP = 8: one tile in eight is waited for.
+template <typename T, int N> constexpr bool p2_ypipe()
+{
+    constexpr int tile = p2_tx2<T, N>() * N * (int)sizeof(typename V2<T>::type);
+    return sizeof(T) == 4 && !P2<N>::R9 && tile > 80 * 1024 && tile + tile / 2 + N * (int)sizeof(typename V2<T>::type) <= 160 * 1024;
+}
+
+template <typename T, int N, int TX, int NP, bool STK>
+__global__ void __launch_bounds__((TX / 2) * (N / 8)) gw_ypass_pipe_kernel(const typename V2<T>::type* __restrict__ W,
+                                                                          typename V2<T>::type* __restrict__ W2,
+                                                                          const typename V2<T>::type* __restrict__ tw,
+                                                                          const LatRef* __restrict__ lat)
+{
+    using T2 = typename V2<T>::type;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    if constexpr (STK) {
+        W = (const T2*)lat[blockIdx.z].W;
+        W2 = (T2*)lat[blockIdx.z].W2;
+    }
+    constexpr int TPT = N / 8, NH = N / 2 + 1, P = half_pitch_c<N>(), H = TX / 2;
+    constexpr int NW = H * TPT / 64, NI = N * TX * (int)sizeof(T2) / (NW * 1024);  // waves; 1 KiB copies of each
+    using L = TiledLayout<N, p2_ztx<T, N>()>;
+    static_assert(sizeof(T) == 4 && TX == 16 && NP % 2 == 0 && N % NP == 0, "pairs of FP32 planes, 128-byte rows");
+    static_assert(L::ZTW % 2 == 0 && P % 2 == 0, "column pairs stay within a tile and a 16-byte line");
+    static_assert(NI * NW * 1024 == N * TX * (int)sizeof(T2), "whole wave copies");
+    __shared__ __align__(16) T2 pf[TX * N];
+    __shared__ __align__(16) T2 s[H * N];
+    __shared__ T2 stw[N];
+    const int b = threadIdx.x % H, j0 = threadIdx.x / H;
+    const int kx = blockIdx.x * TX + 2 * b;
+    const int c = blockIdx.y / (N / NP), z0 = (blockIdx.y % (N / NP)) * NP;
+    const T2* base = W + ((int64_t)c * N + z0) * (int64_t)N * P;
+    // lane l of a wave's copy takes 16 bytes of row l / 8; columns past NH (zeros, or past the row's
+    // last pair: that pair again) are dropped at the stores
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int kc = blockIdx.x * TX + 2 * (lane % 8);
+    const uint32_t off = (lane / 8) * P + (kc < P ? kc : P - 2);
+    auto dma = [&](int q) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int chunk = i * NW + w;
+            __builtin_amdgcn_global_load_lds(
+                (const void __attribute__((address_space(1)))*)(base + (int64_t)q * N * P + chunk * 8 * P + off),
+                (void __attribute__((address_space(3)))*)((__attribute__((address_space(3))) char*)
+                    (__attribute__((address_space(3))) T2*)pf + chunk * 1024), 16, 0, 0);
+        }
+    };
+    for (int i = threadIdx.x; i < N; i += H * TPT) stw[i] = tw[i];
+    dma(0);
+    const P2TwTable<T, N, +1> tws{stw, j0};
+    auto take = [&](int q, T2 (&v0)[8], T2 (&v1)[8]) {
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies have landed
+        lds_sync();                          // and every wave's; the last transform is done with s
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const f32x4 u = *reinterpret_cast<const f32x4*>(pf + (j0 + e * TPT) * TX + 2 * b);
+            v0[e] = T2{u.x, u.y};
+            v1[e] = T2{u.z, u.w};
+        }
+        lds_sync();  // pf read by all: the next copy may start
+        if (q + 1 < NP) dma(q + 1);
+        fft_p2_rb<T, N, +1>(v0, j0, s, H, b, tws);
+        p2_pin(v0);
+        fft_p2_rb<T, N, +1>(v1, j0, s, H, b, tws);
+        p2_pin(v1);
+    };
+#pragma unroll 1
+    for (int q = 0; q < NP; q += 2) {
+        T2 h0[8], h1[8], v0[8], v1[8];
+        take(q, h0, h1);
+        take(q + 1, v0, v1);
+        // padding columns as in gw_ypass_p2_kernel
+        if (kx < L::NT * L::ZTW) {
+            const bool ok0 = kx < NH, ok1 = kx + 1 < NH;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const T2 z = {0, 0};
+                const T2 a = ok0 ? h0[e] : z, aa = ok1 ? h1[e] : z, d = ok0 ? v0[e] : z, dd = ok1 ? v1[e] : z;
+                *reinterpret_cast<f32x4*>(W2 + L::idx(c, z0 + q, j0 + e * TPT, kx)) = f32x4{a.x, a.y, aa.x, aa.y};
+                *reinterpret_cast<f32x4*>(W2 + L::idx(c, z0 + q + 1, j0 + e * TPT, kx)) = f32x4{d.x, d.y, dd.x, dd.y};
+            }
+        }
+    }
+}
+
 // Polarization geometry of one wavevector: z = nz/|n| and r = |n_xy|/|n| (one reciprocal; 0 at k = 0,
 // which is zeroed after the projection), rho2 = |n_xy|^2 and rho its root.
 template <typename T> __device__ __forceinline__ void z_geom(T rho2, T rho, int nz, T& z, T& r)
@@ -389,7 +482,8 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
     // second LDS tile by the waves' direct global-to-LDS loads (16 B per lane, 1 KiB per wave and
     // instruction) while the previous component is transformed.  The transform then synchronises
     // with lds_sync and reads its twiddles from LDS, so that nothing waits for the copies before
-    // the next component's turn.  512^3 FP32C: 1.62-1.63 -> 1.53-1.54 ms, results bit-identical.
+    // the next component's turn.  512^3 FP32C: 1.62-1.63 -> 1.53-1.54 ms, results bit-identical; 768^3
+    // (its radix-3 step too, which had waited for them) 6.05 -> 5.21 ms.
     constexpr bool DMA = p2_zwide<T, N>();
     __shared__ __attribute__((aligned(16))) T2 pf[DMA ? N * TX : 1];
     const int64_t tilebase = L::idx(0, 0, ky, blockIdx.x * TX);
@@ -446,7 +540,7 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
             for (int e = 0; e < 8; e++) v[e] = ok ? ld_stream(base + (int64_t)(j0 + e * TPT) * zs) : T2{0, 0};
         }
         if (c > 0 && !DMA) __syncthreads();
-        if constexpr (DMA && !P2<N>::R3) fft_p2_rb<T, N, +1>(v, j0, s, TX, b, twl);
+        if constexpr (DMA) fft_p2_rb<T, N, +1>(v, j0, s, TX, b, twl);
         else if constexpr (PTW) fft_p2<T, N, +1>(v, j0, s, TX, b, twr);
         else fft_p2<T, N, +1>(v, j0, s, TX, b, twt);
         {
@@ -1085,9 +1179,9 @@ void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const G
             };
             constexpr int TXP = p2_tx<T, NN>(), TXH = TXP > 1 ? TXP / 2 : 1, TX2 = p2_tx2<T, NN>();
             if constexpr (TX2 > 0) {
+                using LT = TiledLayout<NN, p2_ztx<T, NN>()>;
+                constexpr int cols = LT::NT * LT::ZTW > NN / 2 + 1 ? LT::NT * LT::ZTW : NN / 2 + 1;
                 auto go2 = [&]<int KZ>() {
-                    using L = TiledLayout<NN, p2_ztx<T, NN>()>;
-                    constexpr int cols = L::NT * L::ZTW > NN / 2 + 1 ? L::NT * L::ZTW : NN / 2 + 1;
                     auto g2 = [&]<bool STK>() {
                         hipLaunchKernelGGL((gw_ypass_p2w_kernel<T, NN, TX2, KZ, STK>),
                                            dim3((cols + TX2 - 1) / TX2, 6 * NN / KZ, nlat), dim3((TX2 / 2) * (NN / 8)), 0,
@@ -1097,8 +1191,20 @@ void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const G
                     else g2.template operator()<false>();
                 };
                 if (variant == 1) go.template operator()<TXP, 1>();
-                else if (variant == 2) go2.template operator()<2>();
-                else go2.template operator()<1>();
+                else if (variant == 2) {
+                    if constexpr (p2_ypipe<T, NN>()) {
+                        constexpr int NP = 8;
+                        auto g2 = [&]<bool STK>() {
+                            hipLaunchKernelGGL((gw_ypass_pipe_kernel<T, NN, TX2, NP, STK>),
+                                               dim3((cols + TX2 - 1) / TX2, 6 * NN / NP, nlat), dim3((TX2 / 2) * (NN / 8)), 0,
+                                               s, (const T2*)W, (T2*)W2, (const T2*)tw, lat);
+                        };
+                        if (lat) g2.template operator()<true>();
+                        else g2.template operator()<false>();
+                    } else {
+                        go2.template operator()<2>();
+                    }
+                } else go2.template operator()<1>();
             } else {
                 if (variant == 1) go.template operator()<TXH, 1>();
                 else if (variant == 2) go.template operator()<TXP, 2>();
