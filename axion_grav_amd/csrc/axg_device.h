@@ -209,10 +209,13 @@ __device__ __forceinline__ float comp_put(double x, short& lo)
 // accumulators) moves with non-temporal loads and stores, which leave L2 to the re-read halo
 // rows of phi.  Measured at 512^3 FP32C: fused pass 2.49 -> 2.35 ms, y pass 1.40 -> 1.34 ms,
 // z pass 1.65 -> 1.62 ms, step 5.62 -> 5.38 ms (same GPU, results bit-identical).
-template <typename T2>
+// NT false: ordinary accesses, for the passes of a lattice that the last-level cache holds (p2_stream).
+template <bool NT = true, typename T2>
 __device__ __forceinline__ T2 ld_stream(const T2* p)
 {
-    if constexpr (sizeof(T2) == 8) {
+    if constexpr (!NT) {
+        return *p;
+    } else if constexpr (sizeof(T2) == 8) {
         typedef float v2 __attribute__((ext_vector_type(2)));
         const v2 w = __builtin_nontemporal_load(reinterpret_cast<const v2*>(p));
         return T2{w.x, w.y};
@@ -223,16 +226,32 @@ __device__ __forceinline__ T2 ld_stream(const T2* p)
     }
 }
 
-template <typename T2>
+template <bool NT = true, typename T2>
 __device__ __forceinline__ void st_stream(T2* p, T2 v)
 {
-    if constexpr (sizeof(T2) == 8) {
+    if constexpr (!NT) {
+        *p = v;
+    } else if constexpr (sizeof(T2) == 8) {
         typedef float v2 __attribute__((ext_vector_type(2)));
         __builtin_nontemporal_store(v2{v.x, v.y}, reinterpret_cast<v2*>(p));
     } else {
         typedef double v2 __attribute__((ext_vector_type(2)));
         __builtin_nontemporal_store(v2{v.x, v.y}, reinterpret_cast<v2*>(p));
     }
+}
+
+// Whether the passes of a single lattice stream their once-touched data.  They do not for FP32 storage where
+// all that a step touches (three fields with their residuals, the six transformed sources twice and the
+// four accumulators: eleven fields' worth) stays in the 256 MiB last-level cache from pass to pass, which
+// non-temporal accesses go past: per step 128^3 FP32C 94.5 -> 74.3 us, FP32 86 -> 68, 96^3 FP32C 55.7 -> 47.2,
+// 72^3 39.7 -> 35.6; only the loads or only the stores cached: 92 and 87 us at 128^3.  Beyond it cached
+// accesses cost (144^3 FP64 9 %, a mixed batch's stacks together 6 %), and where the set fits the eight
+// 4 MiB L2s the stores' write-back at each kernel's end does (64^3 FP32C 22.7 -> 24.1 us).  FP64 gains
+// nothing from it (96^3 78.7 -> 77.6 us, 72^3 36.9 -> 38.2).
+template <typename T, int N> constexpr bool p2_stream()
+{
+    const int64_t set = (int64_t)N * N * N * (11 * (int64_t)sizeof(typename V2<T>::type) + 12);
+    return sizeof(T) == 8 || set <= (int64_t)32 << 20 || set > (int64_t)240 << 20;
 }
 
 template <typename T, bool COMP>

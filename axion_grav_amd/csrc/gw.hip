@@ -120,6 +120,7 @@ __global__ void __launch_bounds__((TX * (N / 8))) gw_ypass_p2_kernel(const typen
                                                                     const LatRef* __restrict__ lat)
 {
     using T2 = typename V2<T>::type;
+    constexpr bool NT = STK || p2_stream<T, N>();
     if constexpr (STK) {
         // stacked launch: this block's lattice in blockIdx.z
         W = (const T2*)lat[blockIdx.z].W;
@@ -138,7 +139,7 @@ __global__ void __launch_bounds__((TX * (N / 8))) gw_ypass_p2_kernel(const typen
     for (int q = 0; q < KZ; q++) {
         const T2* base = W + ((int64_t)c * N + z0 + q) * (int64_t)N * P + kx;
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[q][e] = ok ? ld_stream(base + (int64_t)(j0 + e * TPT) * P) : T2{0, 0};
+        for (int e = 0; e < 8; e++) v[q][e] = ok ? ld_stream<NT>(base + (int64_t)(j0 + e * TPT) * P) : T2{0, 0};
     }
     // twiddles read inside the stages (measured: no faster with them held in registers)
 #pragma unroll
@@ -387,7 +388,7 @@ template <typename T> __device__ __forceinline__ void z_phase(int64_t n2, const 
 // The updates of grav_waves.f90:239-242 on the accumulators' old values a11, a22, a12 (and a21(),
 // which the index quirk discards) of one wavevector, written to A + m * ms; d6 is the transformed
 // (3,3) source.
-template <typename T, typename F>
+template <typename T, bool NT, typename F>
 __device__ __forceinline__ void z_update(typename V2<T>::type* __restrict__ A, int64_t ms, const GwStepScalars& g, T dw, T cq,
                                          T sq, int64_t rho2, int64_t n2, typename V2<T>::type sp, typename V2<T>::type sn,
                                          typename V2<T>::type d6, typename V2<T>::type a11, typename V2<T>::type a22,
@@ -397,21 +398,21 @@ __device__ __forceinline__ void z_update(typename V2<T>::type* __restrict__ A, i
     using T2 = typename V2<T>::type;
     const T2 SP = {sp.x * dw, sp.y * dw};
     const T2 SN = {sn.x * dw, sn.y * dw};
-    st_stream(A, T2{a11.x + cq * SP.x, a11.y + cq * SP.y});
-    st_stream(A + 3 * ms, T2{a22.x + sq * SN.x, a22.y + sq * SN.y});
+    st_stream<NT>(A, T2{a11.x + cq * SP.x, a11.y + cq * SP.y});
+    st_stream<NT>(A + 3 * ms, T2{a22.x + sq * SN.x, a22.y + sq * SN.y});
     if (!g.fix_swap) {
         T2 r12 = {a12.x + (sq * SP.x + cq * SN.x), a12.y + (sq * SP.y + cq * SN.y)};
         const T n6 = n2 > 0 ? ((T)rho2 / (T)n2) / 2 * dw : (T)0;  // pol_33 dw = r^2/2 dw
-        st_stream(A + 2 * ms, r12);
-        st_stream(A + ms, T2{r12.x - cq * (n6 * d6.x), r12.y - cq * (n6 * d6.y)});
+        st_stream<NT>(A + 2 * ms, r12);
+        st_stream<NT>(A + ms, T2{r12.x - cq * (n6 * d6.x), r12.y - cq * (n6 * d6.y)});
     } else {
         const T2 a21 = a21_old();
-        st_stream(A + ms, T2{a21.x + sq * SP.x, a21.y + sq * SP.y});
-        st_stream(A + 2 * ms, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
+        st_stream<NT>(A + ms, T2{a21.x + sq * SP.x, a21.y + sq * SP.y});
+        st_stream<NT>(A + 2 * ms, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
     }
 }
 
-template <typename T, int N>
+template <typename T, int N, bool NT>
 __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel(const typename V2<T>::type* __restrict__ W,
                                                                            typename V2<T>::type* __restrict__ A,
                                                                            const typename V2<T>::type* __restrict__ tw,
@@ -525,7 +526,7 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
             if (c + 1 < 6) {
                 const T2* base = W + (c + 1) * cst + tile0;
 #pragma unroll
-                for (int e = 0; e < 8; e++) nxt[e] = ok ? ld_stream(base + (int64_t)(j0 + e * TPT) * zs) : T2{0, 0};
+                for (int e = 0; e < 8; e++) nxt[e] = ok ? ld_stream<NT>(base + (int64_t)(j0 + e * TPT) * zs) : T2{0, 0};
             }
         } else if constexpr (DMA) {
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's copies have landed
@@ -537,7 +538,7 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
         } else {
             const T2* base = W + c * cst + tile0;
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = ok ? ld_stream(base + (int64_t)(j0 + e * TPT) * zs) : T2{0, 0};
+            for (int e = 0; e < 8; e++) v[e] = ok ? ld_stream<NT>(base + (int64_t)(j0 + e * TPT) * zs) : T2{0, 0};
         }
         if (c > 0 && !DMA) __syncthreads();
         if constexpr (DMA) fft_p2_rb<T, N, +1>(v, j0, s, TX, b, twl);
@@ -607,18 +608,18 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
         const T2 SN = {sn[e].x * dw, sn[e].y * dw};
         const int64_t ai = tile0 + (int64_t)kz * zs;
         // the accumulators are streamed: each is read and written once per step
-        T2 a11 = ld_stream(A + ai), a22 = ld_stream(A + 3 * ms + ai), a12 = ld_stream(A + 2 * ms + ai);
-        st_stream(A + ai, T2{a11.x + cq * SP.x, a11.y + cq * SP.y});
-        st_stream(A + 3 * ms + ai, T2{a22.x + sq * SN.x, a22.y + sq * SN.y});
+        T2 a11 = ld_stream<NT>(A + ai), a22 = ld_stream<NT>(A + 3 * ms + ai), a12 = ld_stream<NT>(A + 2 * ms + ai);
+        st_stream<NT>(A + ai, T2{a11.x + cq * SP.x, a11.y + cq * SP.y});
+        st_stream<NT>(A + 3 * ms + ai, T2{a22.x + sq * SN.x, a22.y + sq * SN.y});
         if (!g.fix_swap) {
             T2 r12 = {a12.x + (sq * SP.x + cq * SN.x), a12.y + (sq * SP.y + cq * SN.y)};
             const T n6 = n2 > 0 ? ((T)rho2 / (T)n2) / 2 * dw : (T)0;  // pol_33 dw = r^2/2 dw
-            st_stream(A + 2 * ms + ai, r12);
-            st_stream(A + ms + ai, T2{r12.x - cq * (n6 * v[e].x), r12.y - cq * (n6 * v[e].y)});
+            st_stream<NT>(A + 2 * ms + ai, r12);
+            st_stream<NT>(A + ms + ai, T2{r12.x - cq * (n6 * v[e].x), r12.y - cq * (n6 * v[e].y)});
         } else {
-            T2 a21 = ld_stream(A + ms + ai);
-            st_stream(A + ms + ai, T2{a21.x + sq * SP.x, a21.y + sq * SP.y});
-            st_stream(A + 2 * ms + ai, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
+            T2 a21 = ld_stream<NT>(A + ms + ai);
+            st_stream<NT>(A + ms + ai, T2{a21.x + sq * SP.x, a21.y + sq * SP.y});
+            st_stream<NT>(A + 2 * ms + ai, T2{a12.x + cq * SN.x, a12.y + cq * SN.y});
         }
         __builtin_amdgcn_sched_barrier(0);  // keep the k-points' loads from piling up in registers
     }
@@ -644,7 +645,7 @@ template <typename T, int N> constexpr bool p2_zpar()
 
 constexpr int64_t ZPAR_WAVES = 8192;  // 256 CUs x 4 SIMDs x 8 waves
 
-template <typename T, int N>
+template <typename T, int N, bool NT>
 __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel(
     const typename V2<T>::type* __restrict__ W, typename V2<T>::type* __restrict__ A,
     const typename V2<T>::type* __restrict__ tw, GwStepScalars g, StepRef sr, const LatRef* __restrict__ lat)
@@ -661,8 +662,8 @@ __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel
     }
     using L = TiledLayout<N, p2_ztx<T, N>()>;
     using T2 = typename V2<T>::type;
-    constexpr int TX = p2_ztx<T, N>(), TPT = N / 8, NH = N / 2 + 1, NT = p2_zpar_threads<T, N>(), TILE = N * TX;
-    constexpr int KPT = (TILE + NT - 1) / NT;
+    constexpr int TX = p2_ztx<T, N>(), TPT = N / 8, NH = N / 2 + 1, NTH = p2_zpar_threads<T, N>(), TILE = N * TX;
+    constexpr int KPT = (TILE + NTH - 1) / NTH;
     __shared__ T2 s[6 * TILE];
     const int c = threadIdx.x / (TX * TPT), lt = threadIdx.x % (TX * TPT);
     const int b = lt % TX, j0 = lt / TX;
@@ -678,7 +679,7 @@ __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel
     T2 a11[KPT], a22[KPT], a12[KPT], a21[KPT];
 #pragma unroll
     for (int i = 0; i < KPT; i++) {
-        const int t = threadIdx.x + i * NT;
+        const int t = threadIdx.x + i * NTH;
         if (t < TILE && kx0 + t % TX < NH) {
             a11[i] = A[tile0 + t];
             a22[i] = A[3 * ms + tile0 + t];
@@ -696,7 +697,7 @@ __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel
     const T dw = (T)g.dw;
 #pragma unroll
     for (int i = 0; i < KPT; i++) {
-        const int t = threadIdx.x + i * NT;
+        const int t = threadIdx.x + i * NTH;
         if (t >= TILE) break;
         const int kz = t / TX, kx = kx0 + t % TX;
         if (kx >= NH) {
@@ -721,7 +722,7 @@ __global__ void __launch_bounds__((p2_zpar_threads<T, N>())) gw_zpass_par_kernel
         if (n2 == 0) sp = sn = T2{0, 0};  // k = 0: pol = 0
         T cq, sq;
         z_phase<T>(n2, g, cq, sq);
-        z_update<T>(A + tile0 + t, ms, g, dw, cq, sq, rho2, n2, sp, sn, d, a11[i], a22[i], a12[i], [&] { return a21[i]; });
+        z_update<T, NT>(A + tile0 + t, ms, g, dw, cq, sq, rho2, n2, sp, sn, d, a11[i], a22[i], a12[i], [&] { return a21[i]; });
     }
 }
 
@@ -753,7 +754,7 @@ __device__ __forceinline__ void pol_vec(int nx, int ny, int nz, typename V2<T>::
 // gw_zpass_p2_kernel with the projection and update of gw_zpass_acc_kernel (each component of qhat
 // divided by |n|, the update in FP64), which these sizes' accumulators have been made with.  The
 // polarisation vectors are formed once per wavevector.
-template <int N>
+template <int N, bool NT>
 __global__ void __launch_bounds__((p2_ztx<float, N>() * (N / 8))) gw_zpass_p9_kernel(const float2* __restrict__ W,
                                                                               float2* __restrict__ A,
                                                                               const float2* __restrict__ tw,
@@ -784,7 +785,7 @@ __global__ void __launch_bounds__((p2_ztx<float, N>() * (N / 8))) gw_zpass_p9_ke
     float pz[8], pr[8], pc[8], ps[8];  // qz, r, cos and sin of the azimuth, per wavevector
 #pragma unroll
     for (int e = 0; e < 8; e++) {
-        nxt[e] = ok ? ld_stream(W + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
+        nxt[e] = ok ? ld_stream<NT>(W + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
         sp[e] = sn[e] = float2{0, 0};
     }
 #pragma unroll
@@ -803,7 +804,7 @@ __global__ void __launch_bounds__((p2_ztx<float, N>() * (N / 8))) gw_zpass_p9_ke
         if (c + 1 < 6) {
 #pragma unroll
             for (int e = 0; e < 8; e++)
-                nxt[e] = ok ? ld_stream(W + (c + 1) * ms + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
+                nxt[e] = ok ? ld_stream<NT>(W + (c + 1) * ms + tile0 + (int64_t)(j0 + e * TPT) * TX) : float2{0, 0};
         }
         if (c > 0) __syncthreads();
         fft_p2<float, N, +1>(v, j0, s, TX, b, tws);
@@ -834,18 +835,18 @@ __global__ void __launch_bounds__((p2_ztx<float, N>() * (N / 8))) gw_zpass_p9_ke
         const double2 SP = {(double)sp[e].x * dw, (double)sp[e].y * dw};
         const double2 SN = {(double)sn[e].x * dw, (double)sn[e].y * dw};
         float2* a = A + tile0 + (int64_t)kz * TX;
-        const float2 a11 = ld_stream(a), a12 = ld_stream(a + 2 * ms), a22 = ld_stream(a + 3 * ms);
-        st_stream(a, float2{(float)((double)a11.x + cq * SP.x), (float)((double)a11.y + cq * SP.y)});
-        st_stream(a + 3 * ms, float2{(float)((double)a22.x + sq * SN.x), (float)((double)a22.y + sq * SN.y)});
+        const float2 a11 = ld_stream<NT>(a), a12 = ld_stream<NT>(a + 2 * ms), a22 = ld_stream<NT>(a + 3 * ms);
+        st_stream<NT>(a, float2{(float)((double)a11.x + cq * SP.x), (float)((double)a11.y + cq * SP.y)});
+        st_stream<NT>(a + 3 * ms, float2{(float)((double)a22.x + sq * SN.x), (float)((double)a22.y + sq * SN.y)});
         if (!g.fix_swap) {
             const double2 r12 = {(double)a12.x + (sq * SP.x + cq * SN.x), (double)a12.y + (sq * SP.y + cq * SN.y)};
             const double n6 = n2 > 0 ? ((double)rho2 / (double)n2) / 2 * dw : 0.0;
-            st_stream(a + 2 * ms, float2{(float)r12.x, (float)r12.y});
-            st_stream(a + ms, float2{(float)(r12.x - cq * (n6 * (double)v[e].x)), (float)(r12.y - cq * (n6 * (double)v[e].y))});
+            st_stream<NT>(a + 2 * ms, float2{(float)r12.x, (float)r12.y});
+            st_stream<NT>(a + ms, float2{(float)(r12.x - cq * (n6 * (double)v[e].x)), (float)(r12.y - cq * (n6 * (double)v[e].y))});
         } else {
-            const float2 a21 = ld_stream(a + ms);
-            st_stream(a + ms, float2{(float)((double)a21.x + sq * SP.x), (float)((double)a21.y + sq * SP.y)});
-            st_stream(a + 2 * ms, float2{(float)((double)a12.x + cq * SN.x), (float)((double)a12.y + cq * SN.y)});
+            const float2 a21 = ld_stream<NT>(a + ms);
+            st_stream<NT>(a + ms, float2{(float)((double)a21.x + sq * SP.x), (float)((double)a21.y + sq * SP.y)});
+            st_stream<NT>(a + 2 * ms, float2{(float)((double)a12.x + cq * SN.x), (float)((double)a12.y + cq * SN.y)});
         }
     }
 }
@@ -1229,21 +1230,27 @@ void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A
         constexpr int TXP = p2_ztx<T, NN>();
         if (!TiledLayout<NN, TXP>::matches(L))
             throw Error(AXG_EINVAL, "accumulation layout does not match the z pass tile");
-        if constexpr (sizeof(T) == 4 && P2<NN>::R9) {
-            hipLaunchKernelGGL((gw_zpass_p9_kernel<NN>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
-                               (const float2*)W, (float2*)A, (const float2*)tw, g, sr, lat);
-            return;
-        }
-        if constexpr (p2_zpar<T, NN>()) {
-            constexpr int NT = p2_zpar_threads<T, NN>();
-            if ((int64_t)L.ntile * NN * nlat * (NT / 64) <= ZPAR_WAVES) {
-                hipLaunchKernelGGL((gw_zpass_par_kernel<T, NN>), dim3(L.ntile, NN, nlat), dim3(NT), 0, s, (const T2*)W,
-                                   (T2*)A, (const T2*)tw, g, sr, lat);
+        auto go = [&]<bool NT>() {
+            if constexpr (sizeof(T) == 4 && P2<NN>::R9) {
+                hipLaunchKernelGGL((gw_zpass_p9_kernel<NN, NT>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
+                                   (const float2*)W, (float2*)A, (const float2*)tw, g, sr, lat);
                 return;
             }
-        }
-        hipLaunchKernelGGL((gw_zpass_p2_kernel<T, NN>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
-                           (const T2*)W, (T2*)A, (const T2*)tw, g, sr, lat);
+            if constexpr (p2_zpar<T, NN>()) {
+                constexpr int NTH = p2_zpar_threads<T, NN>();
+                if ((int64_t)L.ntile * NN * nlat * (NTH / 64) <= ZPAR_WAVES) {
+                    hipLaunchKernelGGL((gw_zpass_par_kernel<T, NN, NT>), dim3(L.ntile, NN, nlat), dim3(NTH), 0, s, (const T2*)W,
+                                       (T2*)A, (const T2*)tw, g, sr, lat);
+                    return;
+                }
+            }
+            hipLaunchKernelGGL((gw_zpass_p2_kernel<T, NN, NT>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
+                               (const T2*)W, (T2*)A, (const T2*)tw, g, sr, lat);
+        };
+        // a stack's lattices together do not stay in the cache
+        if constexpr (p2_stream<T, NN>()) go.template operator()<true>();
+        else if (lat) go.template operator()<true>();
+        else go.template operator()<false>();
     });
     if (done) { AXG_HIP(hipGetLastError()); return; }
     int TX = col_width<T>(N);

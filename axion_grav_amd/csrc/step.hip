@@ -255,6 +255,7 @@ __global__ void __launch_bounds__(XR * N) kick_source_xfft_kernel(
 {
 #pragma clang fp contract(off)
     using T2 = typename V2<T>::type;
+    constexpr bool NT = STK || p2_stream<T, N>();
     if constexpr (STK) {
         // stacked launch: this block's lattice, its buffers for this step and its scalars
         const LatRef& L = lat[blockIdx.z];
@@ -353,11 +354,11 @@ __global__ void __launch_bounds__(XR * N) kick_source_xfft_kernel(
             const T2* rowp = s + q * N;
             T2 xk = rowp[kk];
             T2 xm = rowp[ring_neg<N>(kk)];
-            st_stream(wa + kk, T2{(T)0.5 * (xk.x + xm.x), (T)0.5 * (xk.y - xm.y)});
-            st_stream(wa + cs + kk, T2{(T)0.5 * (xk.y + xm.y), (T)0.5 * (xm.x - xk.x)});
+            st_stream<NT>(wa + kk, T2{(T)0.5 * (xk.x + xm.x), (T)0.5 * (xk.y - xm.y)});
+            st_stream<NT>(wa + cs + kk, T2{(T)0.5 * (xk.y + xm.y), (T)0.5 * (xm.x - xk.x)});
         } else {
-            st_stream(wa + kk, T2{0, 0});
-            st_stream(wa + cs + kk, T2{0, 0});
+            st_stream<NT>(wa + kk, T2{0, 0});
+            st_stream<NT>(wa + cs + kk, T2{0, 0});
         }
     }
 }
@@ -452,6 +453,7 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
 {
 #pragma clang fp contract(off)
     using T2 = typename V2<T>::type;
+    constexpr bool NT = STK || p2_stream<T, N>();
     if constexpr (STK) {
         // stacked launch: this block's lattice, its buffers for this step and its scalars
         const LatRef& L = lat[blockIdx.z];
@@ -493,13 +495,13 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
         ld_pair<T, COMP>(phi_in, cphi_in, (int64_t)z * NN + (int64_t)yp * N + x0, b20, b21);
         ld_pair<T, COMP>(phi_in, cphi_in, (int64_t)zm * NN + (int64_t)y * N + x0, z10, z11);
         ld_pair<T, COMP>(phi_in, cphi_in, (int64_t)zp * NN + (int64_t)y * N + x0, z20, z21);
-        ld_pair<T, COMP, true>(pi, cpi, row + x0, p0, p1);
+        ld_pair<T, COMP, NT>(pi, cpi, row + x0, p0, p1);
         double2 f0, f1;
         T2 sa[3], sb[3];
         kick_site<T, P2<N>::R9>(c0, l, c1, b10, b20, z10, z20, p0, f0, sa, k, inv_d, d2, div != 0, dt_drift);
         kick_site<T, P2<N>::R9>(c1, c0, r, b11, b21, z11, z21, p1, f1, sb, k, inv_d, d2, div != 0, dt_drift);
-        st_pair<T, COMP, true>(pi, cpi, row + x0, p0, p1);
-        st_pair<T, COMP, true>(phi_out, cphi_out, row + x0, f0, f1);
+        st_pair<T, COMP, NT>(pi, cpi, row + x0, p0, p1);
+        st_pair<T, COMP, NT>(phi_out, cphi_out, row + x0, f0, f1);
 #pragma unroll
         for (int m = 0; m < 3; m++) {
             CPair<T> v;
@@ -545,11 +547,11 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
             const T2* rowp = s + qq * N;
             T2 xk = rowp[kk];
             T2 xm = rowp[ring_neg<N>(kk)];
-            st_stream(wa + kk, T2{(T)0.5 * (xk.x + xm.x), (T)0.5 * (xk.y - xm.y)});
-            st_stream(wa + cs + kk, T2{(T)0.5 * (xk.y + xm.y), (T)0.5 * (xm.x - xk.x)});
+            st_stream<NT>(wa + kk, T2{(T)0.5 * (xk.x + xm.x), (T)0.5 * (xk.y - xm.y)});
+            st_stream<NT>(wa + cs + kk, T2{(T)0.5 * (xk.y + xm.y), (T)0.5 * (xm.x - xk.x)});
         } else {
-            st_stream(wa + kk, T2{0, 0});
-            st_stream(wa + cs + kk, T2{0, 0});
+            st_stream<NT>(wa + kk, T2{0, 0});
+            st_stream<NT>(wa + cs + kk, T2{0, 0});
         }
     }
 }
