@@ -2064,19 +2064,28 @@ static void gradient_impl(axg_handle* h, double t1, double dt, int32_t nsteps, i
     double2* phibar = h->adj;
     double2* pibar = h->adj + n3;       // pibar ping-pongs with pibar2 across the adjoint kicks
     double2* pibar2 = h->adj + 4 * n3;
-    // the adjoint sources in the storage precision (FP32 for FP32 and FP32C lattices)
-    void* W0 = h->work;
-    void* W1 = h->adj + 2 * n3;
-    void* W2 = h->adj + 3 * n3;
-    auto fft_back = [&](void* d) {
-        launch_fft_rows<T, -1>(h->stream, N, d, (int64_t)N * N, h->plan, h->tw);
-        launch_fft_cols<T, -1>(h->stream, N, d, N, (int64_t)N * N, N, N, h->plan, h->tw);
-        launch_fft_cols<T, -1>(h->stream, N, d, (int64_t)N * N, N, N, N, h->plan, h->tw);
+    // the adjoint sources in the storage precision (FP32 for FP32 and FP32C lattices): two FP64 arrays of
+    // h->adj hold all three in FP32, one after the other, and W1 and W2 in FP64
+    char* wadj = (char*)(h->adj + 2 * n3);
+    const size_t wbytes = (size_t)n3 * sizeof(typename V2<T>::type);
+    void* W0 = sizeof(T) == 4 ? (void*)wadj : h->work;
+    void* W1 = sizeof(T) == 4 ? wadj + wbytes : wadj;
+    void* W2 = (char*)W1 + wbytes;
+    // m adjacent arrays at once, along x (unless the gbar kernel does it: the compile-time sizes), y and
+    // z: an array's transforms alone are launches of 7.5 us at 128^3 (gradient's backward step
+    // 11 -> 7 launches)
+    auto fft_back_m = [&](void* d, int m, bool x) {
+        if (x) launch_fft_rows<T, -1>(h->stream, N, d, (int64_t)m * N * N, h->plan, h->tw);
+        launch_fft_cols<T, -1>(h->stream, N, d, N, (int64_t)N * N, m * N, N, h->plan, h->tw);
+        launch_fft_cols<T, -1>(h->stream, N, d, (int64_t)N * N, n3, m, N * N, h->plan, h->tw);
     };
-    // y and z only: the compile-time sizes do the x transform inside the gbar kernel
-    auto fft_back_yz = [&](void* d) {
-        launch_fft_cols<T, -1>(h->stream, N, d, N, (int64_t)N * N, N, N, h->plan, h->tw);
-        launch_fft_cols<T, -1>(h->stream, N, d, (int64_t)N * N, N, N, N, h->plan, h->tw);
+    auto fft_back = [&](bool x) {
+        if (sizeof(T) == 4) {
+            fft_back_m(W0, 3, x);
+        } else {
+            fft_back_m(W0, 1, x);
+            fft_back_m(W1, 2, x);
+        }
     };
     // (the FP32 storages at N with two factors of three keep the separate x pass, first: their adjoint
     // sources have been rounded in that order)
@@ -2167,16 +2176,12 @@ static void gradient_impl(axg_handle* h, double t1, double dt, int32_t nsteps, i
         g.last = s == nsteps - 1;
         launch_adj_modes<T>(h->stream, N, h->abar, g, W0, W1, W2);
         if (fused_x) {
-            fft_back_yz(W0);
-            fft_back_yz(W1);
-            fft_back_yz(W2);
+            fft_back(false);
             if (!launch_adj_gbar_xfft<T, COMP, T>(h->stream, N, h->phi[h->cur], h->cphi[h->cur], inv_d, W0, W1, W2,
                                                   h->tw))
                 throw Error(AXG_EDEVICE, "gradient: no compile-time transform for this size");
         } else {
-            fft_back(W0);
-            fft_back(W1);
-            fft_back(W2);
+            fft_back(true);
             launch_adj_gbar<T, COMP, T>(h->stream, N, h->phi[h->cur], h->cphi[h->cur], inv_d, W0, W1, W2);
         }
         const KickScalars k = kick_scalars(p, t, dt);
