@@ -489,9 +489,11 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         // storage and the dispatcher's order for FP64; code 0 elsewhere (within 10 % of the best)
         if (N == 512) h->kick_variant = h->fp32 ? 9 : 0;
         else if (N == 128 || N == 256 || N == 384 || N >= 768) h->kick_variant = 8;
-        // the y pass at 768 and 1024 in FP32: two columns per thread over 128-byte lines, two z
-        // planes per block (1024^3: 12.7 ms against 16.5 with one plane, 19.9 for the one-column tile)
-        if (h->fp32 && (N == 768 || N == 1024)) h->ypass_variant = 2;
+        // the y pass from 576 in FP32, and in FP64 at the sizes with two factors of three: two columns per
+        // thread over 128-byte lines, two z planes per block (1024^3 FP32C: 12.7 ms against 16.5 with one plane,
+        // 19.9 for the one-column tile; steps at 576^3 FP32C 11.13 -> 10.70 ms, FP64 19.2 -> 17.7, 648^3
+        // 16.2 -> 15.6 and 30.3 -> 28.5, 864^3 FP32C 49.6 -> 40.1; 768^3 FP64 43.7 -> 47.7, so not there)
+        if (N > 512 && (h->fp32 || N % 9 == 0)) h->ypass_variant = 2;
         // tuning knobs AXG_KICK_VARIANT / AXG_YPASS_VARIANT: initial configurations (axg_tune's codes)
         if (const char* e = getenv("AXG_KICK_VARIANT")) h->kick_variant = atoi(e);
         if (const char* e = getenv("AXG_YPASS_VARIANT")) h->ypass_variant = atoi(e);
