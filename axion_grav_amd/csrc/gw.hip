@@ -504,12 +504,16 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
         }
     };
     // the transform's twiddles in LDS: a twiddle load from global memory would wait (vmcnt, in
-    // issue order) for the copies in flight
-    __shared__ T2 stw[DMA ? N : 1];
-    if constexpr (DMA) {
+    // issue order) for the copies in flight; in FP64, which reads them in the stages, where the table is larger
+    // than 4 KiB (steps 432^3 7.18 -> 6.98 ms, 384^3 4.59 -> 4.49, 288^3 1.953 -> 1.929, 512^3 9.47 -> 9.40;
+    // 192^3 0.501 -> 0.505, 128^3 135.5 -> 136.8 us)
+    constexpr bool LTW = DMA || (sizeof(T) == 8 && N > 256);
+    __shared__ T2 stw[LTW ? N : 1];
+    if constexpr (LTW) {
         for (int i = threadIdx.x; i < N; i += TX * (N / 8)) stw[i] = tw[i];
-        dma(0);
     }
+    if constexpr (DMA) dma(0);
+    else if constexpr (LTW) __syncthreads();
     const P2TwTable<T, N, +1> twl{stw, j0};
     if constexpr (PIPE) {
 #pragma unroll
@@ -543,6 +547,7 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
         if (c > 0 && !DMA) __syncthreads();
         if constexpr (DMA) fft_p2_rb<T, N, +1>(v, j0, s, TX, b, twl);
         else if constexpr (PTW) fft_p2<T, N, +1>(v, j0, s, TX, b, twr);
+        else if constexpr (LTW) fft_p2<T, N, +1>(v, j0, s, TX, b, twl);
         else fft_p2<T, N, +1>(v, j0, s, TX, b, twt);
         {
             // pol_ij d into sp (pol d) and sn (conj(pol) d), (i,j) in the reference's order
