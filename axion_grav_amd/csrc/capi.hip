@@ -486,8 +486,10 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         if (const char* e = getenv("AXG_XFUSE")) h->fuse_x = strcmp(e, "0") != 0;
         // the fused pass's configuration before any axg_tune, from the tuner's picks on MI355X:
         // XCD strips at N = 128, 256, 384, 768 and 1024; at 512 wide blocks with strips for FP32
-        // storage and the dispatcher's order for FP64; code 0 elsewhere (within 10 % of the best)
+        // storage and the dispatcher's order for FP64; wide blocks for FP64 at 192 and 384 (twelve waves
+        // instead of six: steps 0.494 -> 0.467 and 4.52 -> 4.44 ms); code 0 elsewhere (within 10 % of the best)
         if (N == 512) h->kick_variant = h->fp32 ? 9 : 0;
+        else if (!h->fp32 && (N == 192 || N == 384)) h->kick_variant = N == 192 ? 1 : 9;
         else if (N == 128 || N == 256 || N == 384 || N >= 768) h->kick_variant = 8;
         // the y pass from 576 in FP32, and in FP64 at the sizes with two factors of three: two columns per
         // thread over 128-byte lines, two z planes per block (1024^3 FP32C: 12.7 ms against 16.5 with one plane,
