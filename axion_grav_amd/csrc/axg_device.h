@@ -254,6 +254,24 @@ template <typename T, int N> constexpr bool p2_stream()
     return sizeof(T) == 8 || set <= (int64_t)32 << 20 || set > (int64_t)240 << 20;
 }
 
+// Runs f.template operator()<STK, NT>() for a step pass: STK with the buffers from a stack's LatRef table (flat
+// addressing) instead of the arguments (global), NT streamed.  cached: ordinary accesses may be used, as p2_stream
+// has it (StepLoad: not beside other lattices that fill the cache with this one; nor by a stack's, which do).
+template <typename T, int N, typename F> void p2_access(bool stacked, bool cached, F&& f)
+{
+    if (stacked) {
+        f.template operator()<true, true>();
+        return;
+    }
+    if constexpr (!p2_stream<T, N>()) {
+        if (cached) {
+            f.template operator()<false, false>();
+            return;
+        }
+    }
+    f.template operator()<false, true>();
+}
+
 template <typename T, bool COMP>
 __device__ __forceinline__ double2 ldf(const typename V2<T>::type* __restrict__ f, const short2* __restrict__ cf,
                                        int64_t i)

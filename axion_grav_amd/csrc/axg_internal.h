@@ -8,6 +8,7 @@
 
 #include "../../include/axgrav.h"
 #include "axg_device.h"
+#include "step_load.h"
 
 // potential.f90:8 -- the truncated pi used by the reference for every physical constant,
 // bin edge and defect threshold.
@@ -101,10 +102,11 @@ void launch_kick_drift(hipStream_t s, int N, const void* phi_in, void* phi_out, 
                        const StepRef& sr = StepRef{});
 
 // Fused kick + source + x transform + drift for p2_size(N); false (nothing launched) otherwise.
+// cached, here and in the y and z passes: see p2_access.
 template <typename T, bool COMP>
 bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi_out, void* pi, const void* cphi_in,
                              void* cphi_out, void* cpi, void* W, int pitch, const void* tw, const KickScalars& k,
-                             double dspa, double dt_drift, int variant, const StepRef& sr = StepRef{},
+                             double dspa, double dt_drift, int variant, bool cached, const StepRef& sr = StepRef{},
                              const LatRef* lat = nullptr, int nlat = 1);
 
 template <typename T>
@@ -189,11 +191,11 @@ void launch_adj_dot(hipStream_t s, int64_t n3, const void* phi, const void* cphi
 // into W2 in the tiled layout.
 template <typename T>
 void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const GwLayout& L, const FftPlan& plan,
-                     const void* tw, int variant = 0, const LatRef* lat = nullptr, int nlat = 1);
+                     const void* tw, int variant, bool cached, const LatRef* lat = nullptr, int nlat = 1);
 
 template <typename T>
 void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A, const GwLayout& L,
-                         const FftPlan& plan, const void* tw, const GwStepScalars& g,
+                         const FftPlan& plan, const void* tw, const GwStepScalars& g, bool cached,
                          const StepRef& sr = StepRef{}, const LatRef* lat = nullptr, int nlat = 1);
 
 template <typename T>

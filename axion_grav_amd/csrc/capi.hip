@@ -262,6 +262,11 @@ struct axg_handle {
         }
         ev_used = 0;
     }
+    // Bytes a step touches, for its StepLoad.
+    int64_t step_set() const
+    {
+        return step_bytes(n3, t2, comp ? 4 : 0, p.grav_spec && !gs) + (gs ? gs->step_set() : 0);
+    }
     void release()
     {
         if (gs) {
@@ -706,7 +711,7 @@ extern "C" int axg_set_gw_state(axg_handle* h, const double* A, int64_t count)
 // out-of-place kick + drift has not overwritten) into the coarse handle's packed source planes,
 // then the coarse grid's x, y and z passes with dw = tau dtau dv_spa_grav sigma_cr^2.
 template <typename T, bool COMP>
-static void reduced_gw_step(axg_handle* h, double t, double dt)
+static void reduced_gw_step(axg_handle* h, double t, double dt, bool cached)
 {
     axg_handle* g = h->gs;
     h->timed(2, [&] {
@@ -715,7 +720,7 @@ static void reduced_gw_step(axg_handle* h, double t, double dt)
         launch_gw_xpass<double>(g->stream, g->N, g->P, g->src, g->W, g->plan, g->tw);
     });
     h->timed(3, [&] {
-        launch_gw_ypass<double>(g->stream, g->N, g->P, g->W, g->W2, g->L, g->plan, g->tw, g->ypass_variant);
+        launch_gw_ypass<double>(g->stream, g->N, g->P, g->W, g->W2, g->L, g->plan, g->tw, g->ypass_variant, cached);
     });
     GwStepScalars s;
     s.tau = t;
@@ -723,13 +728,13 @@ static void reduced_gw_step(axg_handle* h, double t, double dt)
     s.dwav = g->p.dwav;
     s.fix_swap = g->p.gw_fix_swap;
     const void* wz = g->L.zt ? g->W2 : g->W;
-    h->timed(4, [&] { launch_gw_zpass_acc<double>(g->stream, g->N, g->P, wz, g->A, g->L, g->plan, g->tw, s); });
+    h->timed(4, [&] { launch_gw_zpass_acc<double>(g->stream, g->N, g->P, wz, g->A, g->L, g->plan, g->tw, s, cached); });
 }
 
 // The DKD loop; before_kick(s, t) runs before kick s (0-based) at its time t, when phi has
-// reached t and pi is still the previous kick's.
+// reached t and pi is still the previous kick's.  load: the lattice's, until the steps have run.
 template <typename T, bool COMP, typename Hook>
-static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Hook&& before_kick)
+static void run_steps_hooked(axg_handle* h, const StepLoad& load, double t1, double dt, int32_t nt, Hook&& before_kick)
 {
     const int N = h->N;
     const axg_params& p = h->p;
@@ -744,6 +749,7 @@ static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Ho
             t = t + dt / 2;
         }
         before_kick(it - 1, t);
+        const bool cached = load.fits();
         KickScalars k = kick_scalars(p, t, dt);
         double dtd = (it == nt) ? dt / 2 : dt;
         int nxt = 1 - h->cur;
@@ -753,7 +759,7 @@ static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Ho
             h->timed(1, [&] {
                 fused = launch_kick_source_xfft<T, COMP>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi,
                                                          h->cphi[h->cur], h->cphi[nxt], h->cpi, h->W, h->P, h->tw, k,
-                                                         p.dspa, dtd, h->kick_variant);
+                                                         p.dspa, dtd, h->kick_variant, cached);
             });
         }
         if (!fused) {
@@ -762,11 +768,11 @@ static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Ho
                                            h->cphi[nxt], h->cpi, h->src, k, p.dspa, dtd, lattice_gw);
             });
         }
-        if (p.grav_spec && h->gs) reduced_gw_step<T, COMP>(h, t, dt);
+        if (p.grav_spec && h->gs) reduced_gw_step<T, COMP>(h, t, dt, cached);
         if (lattice_gw) {
             if (!fused) h->timed(2, [&] { launch_gw_xpass<T>(h->stream, N, h->P, h->src, h->W, h->plan, h->tw); });
             h->timed(3, [&] {
-                launch_gw_ypass<T>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, h->ypass_variant);
+                launch_gw_ypass<T>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, h->ypass_variant, cached);
             });
             GwStepScalars g;
             g.tau = t;
@@ -774,7 +780,7 @@ static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Ho
             g.dwav = p.dwav;
             g.fix_swap = p.gw_fix_swap;
             const void* wz = h->L.zt ? h->W2 : h->W;
-            h->timed(4, [&] { launch_gw_zpass_acc<T>(h->stream, N, h->P, wz, h->A, h->L, h->plan, h->tw, g); });
+            h->timed(4, [&] { launch_gw_zpass_acc<T>(h->stream, N, h->P, wz, h->A, h->L, h->plan, h->tw, g, cached); });
         }
         h->cur = nxt;
         t = t + dtd;
@@ -782,14 +788,14 @@ static void run_steps_hooked(axg_handle* h, double t1, double dt, int32_t nt, Ho
 }
 
 template <typename T, bool COMP>
-static void run_steps(axg_handle* h, double t1, double dt, int32_t nt)
+static void run_steps(axg_handle* h, const StepLoad& load, double t1, double dt, int32_t nt)
 {
-    run_steps_hooked<T, COMP>(h, t1, dt, nt, [](int32_t, double) {});
+    run_steps_hooked<T, COMP>(h, load, t1, dt, nt, [](int32_t, double) {});
 }
 
 // One DKD step whose scalars come from the handle's step table, entry *base + sidx: the same
-// kernels as run_steps, so the fields match it bit for bit.  Launches only, so it can be
-// captured into a graph; flips h->cur like a step does.
+// kernels as run_steps, so the fields match it bit for bit; streamed, since a batch's other units run
+// beside it.  Launches only, so it can be captured into a graph; flips h->cur like a step does.
 template <typename T, bool COMP>
 static void table_step(axg_handle* h, int sidx, const int* base)
 {
@@ -802,20 +808,20 @@ static void table_step(axg_handle* h, int sidx, const int* base)
     if (p.grav_spec && h->fuse_x)
         fused = launch_kick_source_xfft<T, COMP>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi, h->cphi[h->cur],
                                                  h->cphi[nxt], h->cpi, h->W, h->P, h->tw, k, p.dspa, 0.0,
-                                                 h->kick_variant, sr);
+                                                 h->kick_variant, false, sr);
     if (!fused)
         launch_kick_drift<T, COMP>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi, h->cphi[h->cur], h->cphi[nxt],
                                    h->cpi, h->src, k, p.dspa, 0.0, p.grav_spec != 0, sr);
     if (p.grav_spec) {
         if (!fused) launch_gw_xpass<T>(h->stream, N, h->P, h->src, h->W, h->plan, h->tw);
-        launch_gw_ypass<T>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, h->ypass_variant);
+        launch_gw_ypass<T>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, h->ypass_variant, false);
         GwStepScalars g;
         g.tau = 0;
         g.dw = 0;
         g.dwav = p.dwav;
         g.fix_swap = p.gw_fix_swap;
         const void* wz = h->L.zt ? h->W2 : h->W;
-        launch_gw_zpass_acc<T>(h->stream, N, h->P, wz, h->A, h->L, h->plan, h->tw, g, sr);
+        launch_gw_zpass_acc<T>(h->stream, N, h->P, wz, h->A, h->L, h->plan, h->tw, g, false, sr);
     }
     h->cur = nxt;
 }
@@ -838,15 +844,15 @@ static void stacked_step(axg_handle* h, const LatRef* lat, int nlat, int sidx, c
     const StepRef sr{nullptr, base, sidx};
     const KickScalars k{};
     if (!launch_kick_source_xfft<T, COMP>(h->stream, h->N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                          nullptr, h->P, h->tw, k, p.dspa, 0.0, h->kick_variant, sr, lat, nlat))
+                                          nullptr, h->P, h->tw, k, p.dspa, 0.0, h->kick_variant, false, sr, lat, nlat))
         throw Error(AXG_EINVAL, "stacked step: no fused pass for this size");
-    launch_gw_ypass<T>(h->stream, h->N, h->P, nullptr, nullptr, h->L, h->plan, h->tw, h->ypass_variant, lat, nlat);
+    launch_gw_ypass<T>(h->stream, h->N, h->P, nullptr, nullptr, h->L, h->plan, h->tw, h->ypass_variant, false, lat, nlat);
     GwStepScalars g;
     g.tau = 0;
     g.dw = 0;
     g.dwav = p.dwav;
     g.fix_swap = p.gw_fix_swap;
-    launch_gw_zpass_acc<T>(h->stream, h->N, h->P, nullptr, nullptr, h->L, h->plan, h->tw, g, sr, lat, nlat);
+    launch_gw_zpass_acc<T>(h->stream, h->N, h->P, nullptr, nullptr, h->L, h->plan, h->tw, g, false, sr, lat, nlat);
 }
 
 static void stacked_step_any(axg_handle* h, const LatRef* lat, int nlat, int sidx, const int* base)
@@ -858,9 +864,10 @@ static void stacked_step_any(axg_handle* h, const LatRef* lat, int nlat, int sid
 
 static void advance(axg_handle* h, double t1, double dt, int32_t nt)
 {
-    if (h->comp) run_steps<float, true>(h, t1, dt, nt);
-    else if (h->fp32) run_steps<float, false>(h, t1, dt, nt);
-    else run_steps<double, false>(h, t1, dt, nt);
+    const StepLoad load(h->p.device, h->step_set());
+    if (h->comp) run_steps<float, true>(h, load, t1, dt, nt);
+    else if (h->fp32) run_steps<float, false>(h, load, t1, dt, nt);
+    else run_steps<double, false>(h, load, t1, dt, nt);
     h->have_flags = false;
     h->have_plaq = false;
     h->have_spec = false;
@@ -948,13 +955,13 @@ extern "C" int axg_tune(axg_handle* h, int32_t reps, int32_t* variant, double* m
                 if (h->comp)
                     launch_kick_source_xfft<float, true>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi,
                                                          h->cphi[h->cur], h->cphi[nxt], h->cpi, h->W, h->P, h->tw, k,
-                                                         h->p.dspa, 1e-3, v);
+                                                         h->p.dspa, 1e-3, v, true);
                 else if (h->fp32)
                     launch_kick_source_xfft<float, false>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi, nullptr,
-                                                          nullptr, nullptr, h->W, h->P, h->tw, k, h->p.dspa, 1e-3, v);
+                                                          nullptr, nullptr, h->W, h->P, h->tw, k, h->p.dspa, 1e-3, v, true);
                 else
                     launch_kick_source_xfft<double, false>(h->stream, N, h->phi[h->cur], h->phi[nxt], h->pi, nullptr,
-                                                           nullptr, nullptr, h->W, h->P, h->tw, k, h->p.dspa, 1e-3, v);
+                                                           nullptr, nullptr, h->W, h->P, h->tw, k, h->p.dspa, 1e-3, v, true);
             });
             if (ms && iv < nms) ms[iv] = avg;
             if (avg < best) {
@@ -971,8 +978,8 @@ extern "C" int axg_tune(axg_handle* h, int32_t reps, int32_t* variant, double* m
         if (h->L.zt) {
             for (int yv = 0; yv < 3; yv++) {
                 const double avg = time_avg([&] {
-                    if (h->fp32) launch_gw_ypass<float>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, yv);
-                    else launch_gw_ypass<double>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, yv);
+                    if (h->fp32) launch_gw_ypass<float>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, yv, true);
+                    else launch_gw_ypass<double>(h->stream, N, h->P, h->W, h->W2, h->L, h->plan, h->tw, yv, true);
                 });
                 if (ms && nv + yv < nms) ms[nv + yv] = avg;
                 if (avg < ybest) {
@@ -1957,6 +1964,9 @@ extern "C" int axg_batch_advance(axg_handle* const* hs, int32_t n, double t1, do
         AXG_HIP(hipMemcpyAsync(h0->stepbase, &zero, sizeof zero, hipMemcpyHostToDevice, h0->stream));
         AXG_HIP(hipStreamSynchronize(h0->stream));
         int* base = h0->stepbase;
+        int64_t set = 0;
+        for (int i = 0; i < n; i++) set += hs[i]->step_set();
+        const StepLoad load(h0->p.device, set);
         auto step_unit = [&](const Unit& u, int sidx) {
             if (u.stacked) stacked_step_any(hs[u.idx[0]], h0->latref + u.off, (int)u.idx.size(), sidx, base);
             else table_step_any(hs[u.idx[0]], sidx, base);
@@ -2121,7 +2131,8 @@ static void gradient_impl(axg_handle* h, double t1, double dt, int32_t nsteps, i
     AXG_HIP(hipMemsetAsync(h->A, 0, (size_t)4 * h->L.comp() * fsz, h->stream));
     save(J_INIT);
     std::vector<double> ts(nsteps);
-    run_steps_hooked<T, COMP>(h, t1, dt, nsteps, [&](int32_t s, double t) {
+    const StepLoad steps(h->p.device, h->step_set());
+    run_steps_hooked<T, COMP>(h, steps, t1, dt, nsteps, [&](int32_t s, double t) {
         ts[s] = t;
         if (s % K == 0) save(s / K);
     });

@@ -113,14 +113,13 @@ __global__ void __launch_bounds__((p2_tx<T, N>() * (N / 8))) fft_cols_p2_kernel(
 // planes are transformed one after the other through the same LDS tile, and their outputs for
 // one (ky, kx) are adjacent tile rows, stored back to back (KZ = 2 turns the 64-byte rows of
 // 8-column FP32 or 4-column FP64 tiles into whole 128-byte lines).
-template <typename T, int N, int TX, int KZ, bool STK>
+template <typename T, int N, int TX, int KZ, bool STK, bool NT>
 __global__ void __launch_bounds__((TX * (N / 8))) gw_ypass_p2_kernel(const typename V2<T>::type* __restrict__ W,
                                                                     typename V2<T>::type* __restrict__ W2,
                                                                     const typename V2<T>::type* __restrict__ tw,
                                                                     const LatRef* __restrict__ lat)
 {
     using T2 = typename V2<T>::type;
-    constexpr bool NT = STK || p2_stream<T, N>();
     if constexpr (STK) {
         // stacked launch: this block's lattice in blockIdx.z
         W = (const T2*)lat[blockIdx.z].W;
@@ -1185,7 +1184,7 @@ GwLayout gw_layout(int N, bool fp32)
 
 template <typename T>
 void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const GwLayout& L, const FftPlan& plan,
-                     const void* tw, int variant, const LatRef* lat, int nlat)
+                     const void* tw, int variant, bool cached, const LatRef* lat, int nlat)
 {
     using T2 = typename V2<T>::type;
     if (lat && !L.zt) throw Error(AXG_EINVAL, "stacked y pass needs the tiled layout");
@@ -1199,13 +1198,11 @@ void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const G
             // one-column tile.
             // buffers as arguments or from the stack's LatRef table (global or flat addressing)
             auto go = [&]<int TXP, int KZ>() {
-                auto g1 = [&]<bool STK>() {
-                    hipLaunchKernelGGL((gw_ypass_p2_kernel<T, NN, TXP, KZ, STK>),
+                p2_access<T, NN>(lat != nullptr, cached, [&]<bool STK, bool NT>() {
+                    hipLaunchKernelGGL((gw_ypass_p2_kernel<T, NN, TXP, KZ, STK, NT>),
                                        dim3((NN / 2 + 1 + TXP - 1) / TXP, 6 * NN / KZ, nlat), dim3(TXP * (NN / 8)),
                                        (size_t)NN * TXP * sizeof(T2), s, (const T2*)W, (T2*)W2, (const T2*)tw, lat);
-                };
-                if (lat) g1.template operator()<true>();
-                else g1.template operator()<false>();
+                });
             };
             constexpr int TXP = p2_tx<T, NN>(), TXH = TXP > 1 ? TXP / 2 : 1, TX2 = p2_tx2<T, NN>();
             if constexpr (TX2 > 0) {
@@ -1250,7 +1247,7 @@ void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const G
 
 template <typename T>
 void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A, const GwLayout& L,
-                         const FftPlan& plan, const void* tw, const GwStepScalars& g, const StepRef& sr,
+                         const FftPlan& plan, const void* tw, const GwStepScalars& g, bool cached, const StepRef& sr,
                          const LatRef* lat, int nlat)
 {
     using T2 = typename V2<T>::type;
@@ -1276,10 +1273,8 @@ void launch_gw_zpass_acc(hipStream_t s, int N, int pitch, const void* W, void* A
             hipLaunchKernelGGL((gw_zpass_p2_kernel<T, NN, NT>), dim3(L.ntile, NN, nlat), dim3(TXP * (NN / 8)), 0, s,
                                (const T2*)W, (T2*)A, (const T2*)tw, g, sr, lat);
         };
-        // a stack's lattices together do not stay in the cache
-        if constexpr (p2_stream<T, NN>()) go.template operator()<true>();
-        else if (lat) go.template operator()<true>();
-        else go.template operator()<false>();
+        // (the kernels take a stack's buffers from lat at run time)
+        p2_access<T, NN>(lat != nullptr, cached, [&]<bool STK, bool NT>() { go.template operator()<NT>(); });
     });
     if (done) { AXG_HIP(hipGetLastError()); return; }
     int TX = col_width<T>(N);
@@ -1454,9 +1449,9 @@ void launch_gw_pack(hipStream_t s, int N, const GwLayout& L, void* A, int m, dou
                                          const void*);                                                          \
     template void launch_fft_rows<T, +1>(hipStream_t, int, void*, int64_t, const FftPlan&, const void*);        \
     template void launch_gw_ypass<T>(hipStream_t, int, int, void*, void*, const GwLayout&, const FftPlan&,       \
-                                     const void*, int, const LatRef*, int);                                     \
+                                     const void*, int, bool, const LatRef*, int);                               \
     template void launch_gw_zpass_acc<T>(hipStream_t, int, int, const void*, void*, const GwLayout&,             \
-                                         const FftPlan&, const void*, const GwStepScalars&, const StepRef&,     \
+                                         const FftPlan&, const void*, const GwStepScalars&, bool, const StepRef&, \
                                          const LatRef*, int);                                                   \
     template void launch_gw_bin<T>(hipStream_t, int, const GwLayout&, const void*, const uint16_t*, int64_t, int, double*, \
                                    int, double*);                                                               \

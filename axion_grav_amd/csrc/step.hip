@@ -252,7 +252,7 @@ __device__ __forceinline__ void strip_order(int lin, int& yg, int& z)
 // neighbouring rows of one plane and share their y halo rows in its L2.  REMAP 2 (strips,
 // strip_order): XCD k takes a strip of NG/8 row groups and walks it plane by plane, so its
 // blocks share both the y and the z halo rows.
-template <typename T, bool COMP, int N, int XR, int REMAP, bool STK>
+template <typename T, bool COMP, int N, int XR, int REMAP, bool STK, bool NT>
 __global__ void __launch_bounds__(XR * N) kick_source_xfft_kernel(
     const typename V2<T>::type* __restrict__ phi_in, typename V2<T>::type* __restrict__ phi_out,
     typename V2<T>::type* __restrict__ pi, const short2* __restrict__ cphi_in, short2* __restrict__ cphi_out,
@@ -261,7 +261,6 @@ __global__ void __launch_bounds__(XR * N) kick_source_xfft_kernel(
 {
 #pragma clang fp contract(off)
     using T2 = typename V2<T>::type;
-    constexpr bool NT = STK || p2_stream<T, N>();
     // pi and the drifted phi streamed in FP64 where a single lattice's three fields do not fit the 256 MiB
     // last-level cache (steps 192^3 0.501 -> 0.496 ms, 288^3 1.953 -> 1.922, 512^3 9.47 -> 9.33; 144^3
     // 220 -> 234 us, 96^3 79 -> 84.5)
@@ -461,7 +460,7 @@ __device__ __forceinline__ void st_pair(typename V2<T>::type* __restrict__ f, sh
     }
 }
 
-template <typename T, bool COMP, int N, int XR, bool STRIP, bool STK>
+template <typename T, bool COMP, int N, int XR, bool STRIP, bool STK, bool NT>
 __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
     const typename V2<T>::type* __restrict__ phi_in, typename V2<T>::type* __restrict__ phi_out,
     typename V2<T>::type* __restrict__ pi, const short2* __restrict__ cphi_in, short2* __restrict__ cphi_out,
@@ -470,7 +469,6 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
 {
 #pragma clang fp contract(off)
     using T2 = typename V2<T>::type;
-    constexpr bool NT = STK || p2_stream<T, N>();
     if constexpr (STK) {
         // stacked launch: this block's lattice, its buffers for this step and its scalars
         const LatRef& L = lat[blockIdx.z];
@@ -576,8 +574,8 @@ __global__ void __launch_bounds__(XR * N / 2) kick_source_xfft2_kernel(
 template <typename T, bool COMP>
 bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi_out, void* pi, const void* cphi_in,
                              void* cphi_out, void* cpi, void* W, int pitch, const void* tw, const KickScalars& k,
-                             double dspa, double dt_drift, int variant, const StepRef& sr, const LatRef* lat,
-                             int nlat)
+                             double dspa, double dt_drift, int variant, bool cached, const StepRef& sr,
+                             const LatRef* lat, int nlat)
 {
     using T2 = typename V2<T>::type;
     if (pitch != half_pitch(N)) throw Error(AXG_EINVAL, "fused pass: unexpected half-spectrum pitch");
@@ -588,18 +586,16 @@ bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi
     // configuration (same results; the block shape and order only): bit 0 = wide blocks (twice
     // the rows: 1024 threads), bit 1 = XCD remap by planes (one site per thread only), bit 2 =
     // swap the sites-per-thread choice, bit 3 = XCD strips
-    // a kernel with the buffers as arguments (lat == nullptr) or from the stack's LatRef table: two
-    // instantiations, so that the single-lattice form addresses HBM with global instructions
-    // (reached through the table, the buffers take flat ones)
+    // a kernel with the buffers as arguments (lat == nullptr) or from the stack's LatRef table: instantiated
+    // apart, so that the single-lattice form addresses HBM with global instructions (reached
+    // through the table, the buffers take flat ones)
     auto launch = [&]<int NN, int XR, int RM>() {
-        auto go1 = [&]<bool STK>() {
-            hipLaunchKernelGGL((kick_source_xfft_kernel<T, COMP, NN, XR, RM, STK>), dim3(NN / XR, NN, nlat),
+        p2_access<T, NN>(lat != nullptr, cached, [&]<bool STK, bool NT>() {
+            hipLaunchKernelGGL((kick_source_xfft_kernel<T, COMP, NN, XR, RM, STK, NT>), dim3(NN / XR, NN, nlat),
                                dim3(XR * NN), (size_t)3 * XR * NN * sizeof(T2), s, (const T2*)phi_in, (T2*)phi_out,
                                (T2*)pi, (const short2*)cphi_in, (short2*)cphi_out, (short2*)cpi, (T2*)W, pitch,
                                (const T2*)tw, k, 1.0 / d2, d2, div, dt_drift, sr, lat);
-        };
-        if (lat) go1.template operator()<true>();
-        else go1.template operator()<false>();
+        });
     };
     auto go = [&]<int NN>() {
         constexpr int XR = fused_rows<NN>(), XW = fused_rows_wide<NN>();
@@ -609,15 +605,13 @@ bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi
             const bool two = (sizeof(T) == 4) != ((variant & 4) != 0);
             if (two) {
                 auto launch2 = [&]<int X2, bool ST>() {
-                    auto go2 = [&]<bool STK>() {
-                        hipLaunchKernelGGL((kick_source_xfft2_kernel<T, COMP, NN, X2, ST, STK>), dim3(NN / X2, NN, nlat),
+                    p2_access<T, NN>(lat != nullptr, cached, [&]<bool STK, bool NT>() {
+                        hipLaunchKernelGGL((kick_source_xfft2_kernel<T, COMP, NN, X2, ST, STK, NT>), dim3(NN / X2, NN, nlat),
                                            dim3(X2 * NN / 2), (size_t)3 * X2 * NN * sizeof(T2), s, (const T2*)phi_in,
                                            (T2*)phi_out, (T2*)pi, (const short2*)cphi_in, (short2*)cphi_out,
                                            (short2*)cpi, (T2*)W, (const T2*)tw, k, 1.0 / d2, d2, div, dt_drift, sr,
                                            lat);
-                    };
-                    if (lat) go2.template operator()<true>();
-                    else go2.template operator()<false>();
+                    });
                 };
                 // wide: twice the rows when they divide N and the tile stays within 64 KiB of LDS
                 constexpr int X2W =
@@ -683,7 +677,7 @@ bool launch_kick_source_xfft(hipStream_t s, int N, const void* phi_in, void* phi
                                           const StepRef&);                                                \
     template bool launch_kick_source_xfft<T, C>(hipStream_t, int, const void*, void*, void*, const void*, void*, \
                                                 void*, void*, int, const void*, const KickScalars&, double, double, \
-                                                int, const StepRef&, const LatRef*, int);
+                                                int, bool, const StepRef&, const LatRef*, int);
 AXG_INST_STEP(double, false)
 AXG_INST_STEP(float, false)
 AXG_INST_STEP(float, true)
