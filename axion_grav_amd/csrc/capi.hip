@@ -491,11 +491,19 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         if (const char* e = getenv("AXG_XFUSE")) h->fuse_x = strcmp(e, "0") != 0;
         // the fused pass's configuration before any axg_tune, from the tuner's picks on MI355X:
         // XCD strips at N = 128, 256, 384, 768 and 1024; at 512 wide blocks with strips for FP32
-        // storage and the dispatcher's order for FP64; wide blocks for FP64 at 192 and 384 (twelve waves
-        // instead of six: steps 0.494 -> 0.467 and 4.52 -> 4.44 ms); code 0 elsewhere (within 10 % of the best)
+        // storage and the dispatcher's order for FP64; code 0 elsewhere (within 10 % of the best;
+        // at the sizes with two or more factors of three within 2.3 % of the best of 0, 1, 8 and 9)
         if (N == 512) h->kick_variant = h->fp32 ? 9 : 0;
-        else if (!h->fp32 && (N == 192 || N == 384)) h->kick_variant = N == 192 ? 1 : 9;
         else if (N == 128 || N == 256 || N == 384 || N >= 768) h->kick_variant = 8;
+        // wide blocks with strips in FP64 at N = 3 * 2^k whose three fields pass the 256 MiB last-level cache: the
+        // rows of a block share their y neighbours instead of reading them again, and both blocks are whole
+        // waves, six and twelve (steps 192^3 494 -> 466 us, 384^3 4.35 -> 4.27 ms; 768 has one row either way).
+        // Not in the cache (96^3 79.8 -> 80.8 us), not at 2^k, whose narrow block has eight waves (128^3 137 -> 153,
+        // 256^3 1022 -> 1163 us, 512^3 8.8 -> 10.2 ms), nor where the wide block's last wave is half empty
+        // and its radix-9 barriers wait for thirteen others (216^3 706 -> 748 us, 288^3 1.89 -> 1.99 ms,
+        // 432^3 6.63 -> 7.04)
+        const bool radix3 = p2_size(N) && N % 3 == 0 && N % 9 != 0;
+        if (!h->fp32 && radix3 && h->n3 * 48 > (int64_t)256 << 20) h->kick_variant = 9;
         // the y pass from 576 in FP32, and in FP64 at the sizes with two factors of three: two columns per
         // thread over 128-byte lines, two z planes per block (1024^3 FP32C: 12.7 ms against 16.5 with one plane,
         // 19.9 for the one-column tile; steps at 576^3 FP32C 11.13 -> 10.70 ms, FP64 19.2 -> 17.7, 648^3
