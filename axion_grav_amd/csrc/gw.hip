@@ -27,7 +27,7 @@ template <typename T> int col_width(int N)
 }
 
 
-// ================================================================== N = 2^L, 3 * 2^L specializations
+// ================================================================== compile-time sizes
 // The same three passes with the compile-time radix-8 engine of fft_p2.h: every thread
 // carries 8 elements of one transform in registers, the first load and last store go
 // directly between registers and HBM, and LDS is touched only between stages.
@@ -246,7 +246,7 @@ __global__ void __launch_bounds__((TX / 2) * (N / 8)) gw_ypass_p2w_kernel(const 
 // global-to-LDS loads while the current one is transformed, one column of a thread's pair after the other
 // through half a tile (lds_sync barriers and LDS twiddles, as in the z pass, so that nothing waits
 // for the copies).  Two planes' outputs for one (ky, kx) are adjacent tile rows: the first one's are
-// held and both stored back to back.  768^3 FP32C: 7.58 -> 4.51 ms (5.1 TB/s of its 23.1 GB; the
+// held and both stored back to back.  768^3 FP32C: 7.58 -> 4.51 ms (5 TB/s of its counted 22.4 GB; the
 // two-plane two-column kernel 6.8 with its spills taken out); at 1024 the tile and a half do not fit, at 576 and
 // 648 the radix-9 passes wait for the copies.  NP = 8: one tile in eight is waited for.
 template <typename T, int N> constexpr bool p2_ypipe()
@@ -1238,7 +1238,7 @@ void launch_gw_ypass(hipStream_t s, int N, int pitch, void* W, void* W2, const G
                 else go.template operator()<TXP, 1>();
             }
         });
-        if (!done) throw Error(AXG_EINVAL, "tiled y pass needs N = 2^k or 3 * 2^k");
+        if (!done) throw Error(AXG_EINVAL, "tiled y pass needs a compile-time size");
         AXG_HIP(hipGetLastError());
         return;
     }

@@ -7,7 +7,7 @@
 // beyond the last bin are a fifth of the rows (ky, kz): those rows are neither transformed along x
 // nor read or written by the y pass.
 //
-// A realisation moves 7.1 N^3 complex values instead of 14.5: at 256^3 790 -> 520 us (modes and x 166,
+// A realisation moves 7.5 N^3 complex values (120 B a site) instead of 14.5: at 256^3 790 -> 520 us (modes and x 166,
 // forward y 71, z and mask 113, backward y 73, x and folding 62, binning 37), at 512^3 7.9 -> 5.1
 // ms; a field spectrum at 512^3 9.9 -> 8.1 ms.  The y and x passes run at the rate of a copy, the
 // modes at the rate of their FP64 logarithm, sine and cosine, the z pass, two transforms on one read,

@@ -29,7 +29,7 @@ namespace {
 
 constexpr int STAGE_WORKERS = 7, STAGE_SLOTS = 8;
 constexpr size_t STAGE_CHUNK = (size_t)4 << 20;
-// Two fields out / in, ms, hipMemcpyAsync -> this: 128^3 (16 MiB each) 6.7 / 2.2 -> 4.5 / 2.0, 256^3 51 / 17.5 ->
+// Two fields out / in, ms, hipMemcpyAsync -> this: 128^3 (32 MiB each) 6.7 / 2.2 -> 4.5 / 2.0, 256^3 51 / 17.5 ->
 // 29 / 12 (13 / 12 with a warmed DMA engine), 512^3 410 / 139 -> 95 / 93 (46 GB/s each way); a 512^3
 // flag plane 13 -> 3.4.  Chunks of 2 MiB 109 / 107 and of 1 MiB 143 / 144 at 512^3; 4 workers 103, 11 workers
 // 94.  Below 16 MiB the gain (96^3 3.3 -> 2.5 out, 0.85 -> 1.0 in) does not pay the ring's making, 3 ms once.

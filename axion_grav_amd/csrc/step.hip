@@ -156,8 +156,8 @@ void launch_kick_drift(hipStream_t s, int N, const void* phi_in, void* phi_out, 
 // written to W[2m] and W[2m+1] (the y and z passes follow).  The six source reals per site
 // never reach HBM.
 
-// rows per block: a power of two (it divides N) with blocks of up to 512 threads (measured at
-// 512^3: one row per block beats two by 5-7 % in both precisions), one row when N >= 512; N <= 64 takes
+// rows per block: a divisor of N (p2_rows_div: a power of two, but 6 at 72 and 3 at 144) with blocks of up to 512
+// threads (measured at 512^3: one row per block beats two by 5-7 % in both precisions), one row when N >= 512; N <= 64 takes
 // smaller blocks, whose few hundred would not reach every CU (64 sites to N = 32, 256 to 64: per step
 // 32^3 FP64 15.9 -> 14.0 us, FP32C 14.7 -> 13.0, 16^3 FP64 13.1 -> 12.4, 48^3 FP64 23.6 -> 22.1)
 template <int N> constexpr int fused_rows()

@@ -755,8 +755,8 @@ __global__ void __launch_bounds__(STRING_NT, 3) string_starts_kernel(int N, cons
 
 // Stages two and three: the simplex iterations of the n strings (list null: all of them; else *count strings of the
 // list) up to itmax, one string per lane.  A string still searching goes back to its state and onto
-// pend; the others get their records.  Two waves a SIMD (206 VGPRs); in 168 VGPRs it spills 41 of them
-// and is no faster (512^3, both kernels: 33 ms).
+// pend; the others get their records.  Two waves a SIMD (234 VGPRs); in 168 VGPRs it spills 105 of them
+// (the fits of 785,000 strings at 512^3 47.5 -> 56.3 ms, of 96,000 at 256^3 11.5 -> 13.5).
 static_assert(STRING_NT == 64, "string fit blocks are one wave (see ShrinkLds)");
 template <typename T, bool COMP>
 __global__ void __launch_bounds__(STRING_NT, 2) string_fit_kernel(
