@@ -594,9 +594,12 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
     const int64_t rho2 = (int64_t)nx * nx + (int64_t)ny * ny;
     // the accumulators are streamed, each read and written once per step.  The next k-point's are loaded
     // during the current one's phase and updates (FP64 steps 144^3 229.7 -> 220.1 us, 288^3 2.015 -> 1.960
-    // ms, 128^3 139.5 -> 135.8 us, FP32C 256^3 658 -> 650 us, 512^3 the same), except FP32 ones in the last-level
-    // cache (128^3 FP32C 74.6 -> 76.4 us)
-    constexpr bool AHEAD = NT;
+    // ms, 128^3 139.5 -> 135.8 us, FP32C 256^3 658 -> 650 us), except FP32 ones in the last-level cache
+    // (128^3 FP32C 74.6 -> 76.4 us) and those of blocks over 512 threads, the FP32 sizes from 384, which leave
+    // a CU one block whose waves come to the updates together (this pass, loaded ahead and not: 1024^3 FP32C
+    // 13.25 and 12.36 ms, FP32 13.20 and 12.23; 384^3, 512^3 and 768^3 the same; 192^3 FP32C 122 and 133 us,
+    // 256^3 211 and 216)
+    constexpr bool AHEAD = NT && p2_ztx<T, N>() * (N / 8) <= 512;
     T2 n11, n22, n12;
     auto acc_load = [&](int64_t ai) {
         n11 = ld_stream<NT>(A + ai);
