@@ -324,13 +324,10 @@ void launch_load_field(hipStream_t s, int N, const void* f, const void* cf, doub
 void launch_scatter_modes(hipStream_t s, int N, const int64_t* idx, const double2* val, int64_t nmodes,
                           double2* out);
 
-// in * scale into out
-void launch_scaled_copy(hipStream_t s, int64_t n, const double2* in, double scale, double2* out);
-
 // Copies between the device and a caller's host memory, in stream order after the work on s (staging.hip).
-// copy_to_host returns when the data is there, copy_to_device when pageable host memory may change; page-locked
+// copy_to_host returns when the data is there (wait false: after the next synchronisation of s), copy_to_device when pageable host memory may change; page-locked
 // memory is still being read then, so the entry points synchronise before they return.
-void copy_to_host(int device, hipStream_t s, void* dst, const void* src, size_t bytes);
+void copy_to_host(int device, hipStream_t s, void* dst, const void* src, size_t bytes, bool wait = true);
 void copy_to_device(int device, hipStream_t s, void* dst, const void* src, size_t bytes);
 // One more / one less handle on the device (its pinned chunks go with the last).
 void staging_retain(int device);

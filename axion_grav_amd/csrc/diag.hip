@@ -757,22 +757,9 @@ __global__ void scale_kernel(int64_t n, double2* __restrict__ d, double sc)
     }
 }
 
-__global__ void scaled_copy_kernel(int64_t n, const double2* __restrict__ in, double sc, double2* __restrict__ out)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = double2{in[i].x * sc, in[i].y * sc};
-}
-
-void launch_scaled_copy(hipStream_t s, int64_t n, const double2* in, double scale, double2* out)
-{
-    hipLaunchKernelGGL(scaled_copy_kernel, dim3((unsigned)std::min<int64_t>(65536, (n + 255) / 256)), dim3(256), 0, s, n, in,
-                       scale, out);
-    AXG_HIP(hipGetLastError());
-}
-
 void launch_scale(hipStream_t s, int64_t n, double2* data, double scale)
 {
-    hipLaunchKernelGGL(scale_kernel, dim3(65536), dim3(256), 0, s, n, data, scale);
+    hipLaunchKernelGGL(scale_kernel, dim3((unsigned)std::min<int64_t>(65536, (n + 255) / 256)), dim3(256), 0, s, n, data, scale);
     AXG_HIP(hipGetLastError());
 }
 

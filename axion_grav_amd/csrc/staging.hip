@@ -189,11 +189,11 @@ void staging_release(int device)
     p.give_back();
 }
 
-void copy_to_host(int device, hipStream_t s, void* dst, const void* src, size_t bytes)
+void copy_to_host(int device, hipStream_t s, void* dst, const void* src, size_t bytes, bool wait)
 {
     if (staged(device, s, (char*)dst, (const char*)src, bytes, true)) return;
     AXG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-    AXG_HIP(hipStreamSynchronize(s));
+    if (wait) AXG_HIP(hipStreamSynchronize(s));
 }
 
 void copy_to_device(int device, hipStream_t s, void* dst, const void* src, size_t bytes)
