@@ -272,6 +272,27 @@ template <typename T, int N, typename F> void p2_access(bool stacked, bool cache
     f.template operator()<false, true>();
 }
 
+// The folded power of a transformed row at j = 0..N/2, |amp X(j)|^2 + |amp X(N-j)|^2 (once for j = 0 and N/2): FOLDED
+// it is there already, in the row's first N/2 + 1 reals; otherwise from the row's N complex values.
+template <bool FOLDED> struct SpecPair {
+    double p = 0;
+    __device__ __forceinline__ void load(const double2* row, int, int j) { p = reinterpret_cast<const double*>(row)[j]; }
+    __device__ __forceinline__ double power(double) const { return p; }
+};
+template <> struct SpecPair<false> {
+    double2 a = {0, 0}, b = {0, 0};
+    __device__ __forceinline__ void load(const double2* row, int N, int j)
+    {
+        a = row[j];
+        b = j > 0 && j < N / 2 ? row[N - j] : double2{0, 0};
+    }
+    __device__ __forceinline__ double power(double amp) const
+    {
+        const double ax = a.x * amp, ay = a.y * amp, bx = b.x * amp, by = b.y * amp;
+        return (ax * ax + ay * ay) + (bx * bx + by * by);
+    }
+};
+
 template <typename T, bool COMP>
 __device__ __forceinline__ double2 ldf(const typename V2<T>::type* __restrict__ f, const short2* __restrict__ cf,
                                        int64_t i)

@@ -304,12 +304,13 @@ size_t spec_mask_bytes(int N);
 void launch_spec_mask_bits(hipStream_t s, int N, const int8_t* flags, uint8_t* bits);
 void launch_spec_z_mask(hipStream_t s, int N, double2* data, const uint8_t* bits, const double2* tw);
 void launch_spec_fold_x(hipStream_t s, int N, double2* data, int64_t n2max, double amp, const double2* tw);
-void launch_spec_fold(hipStream_t s, int N, double2* data, double amp);
 
-void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* bin_of_n2, int64_t n2max, int nb,
-                     double* partial, int nwg, double* out);
+// They take the folded power or, folded false (an array transformed by the runtime-plan passes), the transform itself,
+// launch_spec_bin times amp.
+void launch_spec_bin(hipStream_t s, int N, const double2* data, bool folded, double amp, const uint16_t* bin_of_n2,
+                     int64_t n2max, int nb, double* partial, int nwg, double* out);
 
-void launch_n2_hist(hipStream_t s, int N, const double2* data, double* plane_part, double* hist);
+void launch_n2_hist(hipStream_t s, int N, const double2* data, bool folded, double* plane_part, double* hist);
 
 void launch_deconv_mat(hipStream_t s, int nb, int num_cov, int nlq, const double* largeq, const double* mat,
                        const double* dqs, const double* hist, const double* cnt, int64_t nn2, double dwav,

@@ -1497,27 +1497,27 @@ static void fft3d_work(axg_handle* h, double2* d, int sign = +1)
     }
 }
 
-// Folded power of the BACKWARD transform of (mask ? 0 : pi) or, use_pi false, of the window
-// (mask ? 0 : fill), times amp^2, into h->work; the rows beyond n2max are left out.
+// BACKWARD transform of (mask ? 0 : pi) or, use_pi false, of the window (mask ? 0 : fill), into h->work: its folded
+// power times amp^2, the rows beyond n2max left out, at the sizes with compile-time kernels (true), or itself.
 template <typename T, bool COMP>
-static void masked_power(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
+static bool masked_power(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
 {
     const double2* tw = (const double2*)h->tw64;
     if (launch_spec_z_field<T, COMP>(h->stream, h->N, h->pi, h->cpi, h->flags, fill, use_pi, h->work, tw)) {
         launch_spec_y(h->stream, h->N, h->work, +1, n2max < h->nn2 - 1, n2max, tw);
         launch_spec_fold_x(h->stream, h->N, h->work, n2max, amp, tw);
-        return;
+        return true;
     }
     launch_masked_field<T, COMP>(h->stream, h->N, h->pi, h->cpi, h->flags, h->work, fill, use_pi);
     fft3d_work(h, h->work);
-    launch_spec_fold(h->stream, h->N, h->work, amp);
+    return false;
 }
 
-static void masked_power_any(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
+static bool masked_power_any(axg_handle* h, bool use_pi, double fill, double amp, int64_t n2max)
 {
-    if (h->comp) masked_power<float, true>(h, use_pi, fill, amp, n2max);
-    else if (h->fp32) masked_power<float, false>(h, use_pi, fill, amp, n2max);
-    else masked_power<double, false>(h, use_pi, fill, amp, n2max);
+    if (h->comp) return masked_power<float, true>(h, use_pi, fill, amp, n2max);
+    if (h->fp32) return masked_power<float, false>(h, use_pi, fill, amp, n2max);
+    return masked_power<double, false>(h, use_pi, fill, amp, n2max);
 }
 
 // Runs body(lo, hi) over [0, n) split into contiguous ranges on up to 16 host threads (the
@@ -1617,8 +1617,8 @@ extern "C" int axg_field_spectrum(axg_handle* h, double tau, double* qmid, doubl
         const int ncov = nb * (nb + 1) / 2;
         const int nwg = 1024;
         // compute_matrix_deconv (spectrum.f90:358-433): window = dv_spa with mask cells zeroed
-        masked_power_any(h, false, p.dv_spa, 1.0, h->nn2 - 1);
-        launch_n2_hist(h->stream, h->N, h->work, h->d_plane, h->d_hist);
+        const bool fw = masked_power_any(h, false, p.dv_spa, 1.0, h->nn2 - 1);
+        launch_n2_hist(h->stream, h->N, h->work, fw, h->d_plane, h->d_hist);
         double* mat0 = h->red;
         double* tat0 = h->red + ncov;
         require((size_t)2 * ncov * 8 <= h->red_bytes, "reduction scratch too small");
@@ -1629,10 +1629,10 @@ extern "C" int axg_field_spectrum(axg_handle* h, double tau, double* qmid, doubl
         AXG_HIP(hipMemcpyAsync(t0.data(), tat0, ncov * 8, hipMemcpyDeviceToHost, h->stream));
         AXG_HIP(hipStreamSynchronize(h->stream));
         // compute_conv_spec (spectrum.f90:474-563): masked pi -> FFT -> *dv_spa -> binned
-        masked_power_any(h, true, 0.0, p.dv_spa, h->spec_n2max);
+        const bool fp = masked_power_any(h, true, 0.0, p.dv_spa, h->spec_n2max);
         double* out = h->red + (size_t)nwg * 2 * nb;
         require((size_t)(nwg + 1) * 2 * nb * 8 <= h->red_bytes, "reduction scratch too small");
-        launch_spec_bin(h->stream, h->N, h->work, h->spec_bin, h->spec_n2max, nb, h->red, nwg, out);
+        launch_spec_bin(h->stream, h->N, h->work, fp, p.dv_spa, h->spec_bin, h->spec_n2max, nb, h->red, nwg, out);
         std::vector<double> r(2 * nb);
         AXG_HIP(hipMemcpyAsync(r.data(), out, 2 * nb * 8, hipMemcpyDeviceToHost, h->stream));
         AXG_HIP(hipStreamSynchronize(h->stream));
@@ -1748,7 +1748,8 @@ extern "C" int axg_field_covariance(axg_handle* h, uint64_t seed, int32_t min_mc
         }
         for (; iter <= max_mc; iter++) {
             const double2* tw = (const double2*)h->tw64;
-            if (launch_spec_modes_x(h->stream, N, dr, iter, h->spec_bin, h->spec_n2max, d_sig, h->work, tw)) {
+            const bool folded = launch_spec_modes_x(h->stream, N, dr, iter, h->spec_bin, h->spec_n2max, d_sig, h->work, tw);
+            if (folded) {
                 launch_spec_y(h->stream, N, h->work, -1, 1, h->spec_n2max, tw);
                 launch_spec_z_mask(h->stream, N, h->work, h->d_maskbits, tw);
                 launch_spec_y(h->stream, N, h->work, +1, 1, h->spec_n2max, tw);
@@ -1758,9 +1759,8 @@ extern "C" int axg_field_covariance(axg_handle* h, uint64_t seed, int32_t min_mc
                 fft3d_work(h, h->work, -1);
                 launch_mask_zero(h->stream, h->n3, h->flags, h->work);
                 fft3d_work(h, h->work, +1);
-                launch_spec_fold(h->stream, N, h->work, 1.0);
             }
-            launch_spec_bin(h->stream, N, h->work, h->spec_bin, h->spec_n2max, nb, part, nwg, out);
+            launch_spec_bin(h->stream, N, h->work, folded, 1.0, h->spec_bin, h->spec_n2max, nb, part, nwg, out);
             AXG_HIP(hipMemcpyAsync(r.data(), out, 2 * nb * 8, hipMemcpyDeviceToHost, h->stream));
             AXG_HIP(hipStreamSynchronize(h->stream));
             // pow = mat_deconv pow0 - power (dspmv with beta = 1, spectrum.f90:675-677)

@@ -421,7 +421,9 @@ void launch_masked_field(hipStream_t s, int N, const void* pi, const void* cpi, 
 
 // Shell binning over the full spectrum (spectrum.f90:530-556) of the folded power (axg_internal.h): row
 // (ky,kz) holds j = |nx| = 0..N/2, along which the bin is non-decreasing, so every bin is one run
-// of the row.  pow[b] += |.|^2 (times dv_wav on the host), num[b] += 1 per mode.
+// of the row.  pow[b] += |.|^2 (times dv_wav on the host), num[b] += 1 per mode.  FOLDED false: the rows are
+// the runtime-plan passes' and are folded here (in a pass of their own, the histogram's too, a field spectrum
+// at 18^3 to 108^3 took 10 to 20 us more: 36^3 189 -> 204).
 //
 // A wave takes a row at a time, into its own LDS bins: the last element of a run records where the run
 // ends and the lane at its start sums it in order.  No barrier and no other wave is waited for
@@ -441,8 +443,8 @@ static size_t spec_bin_lds(int N, int nb)
     return ((size_t)(2 * nb + N / 2 + 1) * sizeof(double) + (size_t)(N / 2 + 1 + nb) * sizeof(int) + 7) / 8 * 8;
 }
 
-template <int KP>
-__global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __restrict__ d,
+template <int KP, bool FOLDED>
+__global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __restrict__ d, double amp,
                                                        const uint16_t* __restrict__ bin_of_n2, int64_t n2max, int nb,
                                                        double* __restrict__ partial)
 {
@@ -455,7 +457,7 @@ __global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __r
     int* rend = bb + nh;  // nb: one past the last j of bin b's run in the row
     const int64_t NN = (int64_t)N * N;
     for (int b = lane; b < 2 * nb; b += 64) bins[b] = 0;
-    double a[KP];
+    SpecPair<FOLDED> a[KP];
     int bq[KP];
     const int64_t step = (int64_t)gridDim.x * nw;
     // the wave's next row with a binned mode, its values and bins in registers
@@ -465,14 +467,14 @@ __global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __r
             const int ny = wrapn(ky, N), nz = wrapn(kz, N);
             const int64_t m2 = (int64_t)ny * ny + (int64_t)nz * nz;
             if (m2 > n2max) continue;
-            const double* r = (const double*)(d + row * N);
 #pragma unroll
             for (int i = 0; i < KP; i++) {
                 const int j = lane + i * 64;
                 const int64_t n2 = (int64_t)j * j + m2;
                 const bool in = j < nh && n2 <= n2max;
                 bq[i] = in ? bin_of_n2[n2] : 0;
-                a[i] = in ? r[j] : 0.0;
+                a[i] = SpecPair<FOLDED>{};
+                if (in) a[i].load(d + row * N, N, j);
             }
             break;
         }
@@ -484,7 +486,7 @@ __global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __r
         for (int i = 0; i < KP; i++) {
             const int j = lane + i * 64;
             if (j < nh) {
-                v[j] = a[i];
+                v[j] = a[i].power(amp);
                 bb[j] = bq[i];
             }
         }
@@ -525,8 +527,8 @@ __global__ void __launch_bounds__(256) spec_bin_kernel(int N, const double2* __r
     }
 }
 
-void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* bin_of_n2, int64_t n2max, int nb,
-                     double* partial, int nwg, double* out)
+void launch_spec_bin(hipStream_t s, int N, const double2* data, bool folded, double amp, const uint16_t* bin_of_n2,
+                     int64_t n2max, int nb, double* partial, int nwg, double* out)
 {
     const int kp = (N / 2 + 1 + 63) / 64;
     if (kp > 9) throw Error(AXG_EINVAL, "field spectrum: N too large for the binning kernel");
@@ -534,7 +536,12 @@ void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* 
     const size_t per = spec_bin_lds(N, nb);
     const int nw = (int)std::max<size_t>(1, std::min<size_t>(4, 65536 / per));
     auto go = [&]<int KP>() {
-        hipLaunchKernelGGL(spec_bin_kernel<KP>, dim3(nwg), dim3(64 * nw), per * nw, s, N, data, bin_of_n2, n2max, nb, partial);
+        if (folded)
+            hipLaunchKernelGGL((spec_bin_kernel<KP, true>), dim3(nwg), dim3(64 * nw), per * nw, s, N, data, amp, bin_of_n2,
+                               n2max, nb, partial);
+        else
+            hipLaunchKernelGGL((spec_bin_kernel<KP, false>), dim3(nwg), dim3(64 * nw), per * nw, s, N, data, amp, bin_of_n2,
+                               n2max, nb, partial);
     };
     if (kp <= 1) go.template operator()<1>();
     else if (kp == 2) go.template operator()<2>();
@@ -547,7 +554,7 @@ void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* 
     sum_columns(s, partial, nwg, 2 * nb, out);
 }
 
-// Histogram of |W|^2 (its folded power) by n^2 = |n|^2, deterministic: block kz walks its plane by a = |ny|
+// Histogram of |W|^2 (its folded power, or W itself) by n^2 = |n|^2, deterministic: block kz walks its plane by a = |ny|
 // (a = 0 .. N/2, in order).  The rows ky = a and ky = N - a share a, so their values at each
 // folded j = |nx| land on the same m = j^2 + a^2 and are added together first; within one a the
 // j hit distinct m, so the per-plane partial plane[kz][m] needs no atomics.  Each thread loads
@@ -555,6 +562,7 @@ void launch_spec_bin(hipStream_t s, int N, const double2* data, const uint16_t* 
 // hist[n2] = sum over kz (in order) of plane[kz][n2 - nz^2].
 constexpr int N2P_NT = 256, N2P_KPT = 3;  // folded j values per thread: N / 2 + 1 <= 768
 
+template <bool FOLDED>
 __global__ void __launch_bounds__(N2P_NT) n2_plane_kernel(int N, const double2* __restrict__ d,
                                                           double* __restrict__ plane)
 {
@@ -563,17 +571,17 @@ __global__ void __launch_bounds__(N2P_NT) n2_plane_kernel(int N, const double2* 
     const int kz = blockIdx.x;
     double* pp = plane + (int64_t)kz * mm;
     for (int64_t m = threadIdx.x; m < mm; m += blockDim.x) pp[m] = 0;
-    double u[N2P_KPT][2];  // rows a and N - a
+    SpecPair<FOLDED> u[N2P_KPT][2];  // rows a and N - a
     auto fetch = [&](int a) {
-        const double* r1 = (const double*)(d + ((int64_t)kz * N + a) * N);
-        const double* r2 = (const double*)(d + ((int64_t)kz * N + (N - a)) * N);
+        const double2* r1 = d + ((int64_t)kz * N + a) * N;
+        const double2* r2 = d + ((int64_t)kz * N + (N - a)) * N;
         const bool two = a > 0 && a < N / 2;
 #pragma unroll
         for (int i = 0; i < N2P_KPT; i++) {
             const int j = threadIdx.x + i * N2P_NT;
             if (j < nh) {
-                u[i][0] = r1[j];
-                if (two) u[i][1] = r2[j];
+                u[i][0].load(r1, N, j);
+                if (two) u[i][1].load(r2, N, j);
             }
         }
     };
@@ -584,7 +592,7 @@ __global__ void __launch_bounds__(N2P_NT) n2_plane_kernel(int N, const double2* 
         double s[N2P_KPT];
 #pragma unroll
         for (int i = 0; i < N2P_KPT; i++) {
-            s[i] = two ? u[i][0] + u[i][1] : u[i][0];
+            s[i] = two ? u[i][0].power(1.0) + u[i][1].power(1.0) : u[i][0].power(1.0);
         }
         if (a < N / 2) fetch(a + 1);
 #pragma unroll
@@ -617,10 +625,11 @@ __global__ void n2_merge_kernel(int N, const double* __restrict__ plane, double*
     hist[n2] = s;
 }
 
-void launch_n2_hist(hipStream_t s, int N, const double2* data, double* plane_part, double* hist)
+void launch_n2_hist(hipStream_t s, int N, const double2* data, bool folded, double* plane_part, double* hist)
 {
     if (N / 2 + 1 > N2P_KPT * N2P_NT) throw Error(AXG_EINVAL, "field spectrum: N too large for the window histogram");
-    hipLaunchKernelGGL(n2_plane_kernel, dim3(N), dim3(N2P_NT), 0, s, N, data, plane_part);
+    if (folded) hipLaunchKernelGGL(n2_plane_kernel<true>, dim3(N), dim3(N2P_NT), 0, s, N, data, plane_part);
+    else hipLaunchKernelGGL(n2_plane_kernel<false>, dim3(N), dim3(N2P_NT), 0, s, N, data, plane_part);
     AXG_HIP(hipGetLastError());
     int64_t nn2 = (int64_t)3 * (N / 2) * (N / 2) + 1;
     hipLaunchKernelGGL(n2_merge_kernel, dim3((unsigned)((nn2 + 255) / 256)), dim3(256), 0, s, N, plane_part, hist);

@@ -191,20 +191,7 @@ __global__ void __launch_bounds__((p2_tx<double, N>() * (N / 8))) spec_z_field_k
     }
 }
 
-// Folded power of a transformed row X in LDS: |amp X(j)|^2 + |amp X(N-j)|^2 (once for j = 0, N/2).
-__device__ __forceinline__ double folded(const double2* X, int N, int j, double amp)
-{
-    double ax = X[j].x * amp, ay = X[j].y * amp;
-    double p = ax * ax + ay * ay;
-    if (j > 0 && j < N / 2) {
-        ax = X[N - j].x * amp;
-        ay = X[N - j].y * amp;
-        p += ax * ax + ay * ay;
-    }
-    return p;
-}
-
-// BACKWARD transform along x of the rows within n2max and their folded power, N/2 + 1 reals at the
+// BACKWARD transform along x of the rows within n2max and their folded power (SpecPair), N/2 + 1 reals at the
 // beginning of the row's own N complex values.
 template <int N>
 __global__ void __launch_bounds__(p2_rows_per_block<N>() * (N / 8))
@@ -230,26 +217,11 @@ __global__ void __launch_bounds__(p2_rows_per_block<N>() * (N / 8))
 #pragma unroll
         for (int i = 0; i < 5; i++) {
             const int j = j0 + i * TPT;
-            if (j <= N / 2) reinterpret_cast<double*>(base)[j] = folded(sr, N, j, amp);
+            if (j > N / 2) continue;
+            SpecPair<false> p;
+            p.load(sr, N, j);
+            reinterpret_cast<double*>(base)[j] = p.power(amp);
         }
-    }
-}
-
-// The folding by itself, for rows transformed by the runtime-plan passes: one row a block, in place.
-__global__ void __launch_bounds__(256) spec_fold_kernel(int N, double2* __restrict__ data, double amp)
-{
-    double2* X = data + (int64_t)blockIdx.x * N;
-    double p[3];
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const int j = threadIdx.x + i * 256;
-        p[i] = j <= N / 2 ? folded(X, N, j, amp) : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const int j = threadIdx.x + i * 256;
-        if (j <= N / 2) reinterpret_cast<double*>(X)[j] = p[i];
     }
 }
 
@@ -326,13 +298,6 @@ void launch_spec_fold_x(hipStream_t s, int N, double2* data, int64_t n2max, doub
                            tw);
     });
     if (!done) throw Error(AXG_EINVAL, "spectrum passes need a compile-time size");
-    AXG_HIP(hipGetLastError());
-}
-
-void launch_spec_fold(hipStream_t s, int N, double2* data, double amp)
-{
-    if (N / 2 + 1 > 3 * 256) throw Error(AXG_EINVAL, "field spectrum: N too large for the folding kernel");
-    hipLaunchKernelGGL(spec_fold_kernel, dim3(N * N), dim3(256), 0, s, N, data, amp);
     AXG_HIP(hipGetLastError());
 }
 
