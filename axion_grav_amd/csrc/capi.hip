@@ -126,6 +126,7 @@ struct axg_handle {
     int cur = 0;
     bool fuse_x = true;      // x transform fused into the stencil pass when p2_size(N)
     int kick_variant = 0;    // configuration of the fused pass (axg_tune codes; set per size at creation)
+    int kick_variant_stack = 0;  // in a batch's stacked launches
     int ypass_variant = 0;   // configuration of the y pass (axg_tune; 0 = 128-byte column tiles)
     // diagnostics
     uint16_t* gw_bin = nullptr;
@@ -494,13 +495,15 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         // at the sizes with two or more factors of three within 2.3 % of the best of 0, 1, 8 and 9)
         if (N == 512) h->kick_variant = h->fp32 ? 9 : 0;
         else if (N == 128 || N == 256 || N == 384 || N >= 768) h->kick_variant = 8;
-        // wide blocks with strips in FP64 at N = 3 * 2^k whose three fields pass the 256 MiB last-level cache: the
-        // rows of a block share their y neighbours instead of reading them again, and both blocks are whole
-        // waves, six and twelve (steps 192^3 494 -> 466 us, 384^3 4.35 -> 4.27 ms; 768 has one row either way).
+        h->kick_variant_stack = h->kick_variant;
+        // a single lattice: wide blocks with strips in FP64 at N = 3 * 2^k whose three fields pass the 256 MiB
+        // last-level cache: the rows of a block share their y neighbours instead of reading them again, and both
+        // blocks are whole waves, six and twelve (steps 192^3 494 -> 466 us, 384^3 4.35 -> 4.27 ms; 768 has one row either way).
         // Not in the cache (96^3 79.8 -> 80.8 us), not at 2^k, whose narrow block has eight waves (128^3 137 -> 153,
         // 256^3 1022 -> 1163 us, 512^3 8.8 -> 10.2 ms), nor where the wide block's last wave is half empty
         // and its radix-9 barriers wait for thirteen others (216^3 706 -> 748 us, 288^3 1.89 -> 1.99 ms,
-        // 432^3 6.63 -> 7.04)
+        // 432^3 6.63 -> 7.04).  Not in a batch's stacks, of which two run at once (batches of 192^3 493 and 554 us
+        // a lattice step narrow and wide, 384^3 4.68 and 5.04 ms)
         const bool radix3 = p2_size(N) && N % 3 == 0 && N % 9 != 0;
         if (!h->fp32 && radix3 && h->n3 * 48 > (int64_t)256 << 20) h->kick_variant = 9;
         // the y pass from 576 in FP32, and in FP64 at the sizes with two factors of three: two columns per
@@ -509,7 +512,7 @@ extern "C" int axg_create(const axg_params* pin, axg_handle** out)
         // 16.2 -> 15.6 and 30.3 -> 28.5, 864^3 FP32C 49.6 -> 40.1; 768^3 FP64 43.7 -> 47.7, so not there)
         if (N > 512 && (h->fp32 || N % 9 == 0)) h->ypass_variant = 2;
         // tuning knobs AXG_KICK_VARIANT / AXG_YPASS_VARIANT: initial configurations (axg_tune's codes)
-        if (const char* e = getenv("AXG_KICK_VARIANT")) h->kick_variant = atoi(e);
+        if (const char* e = getenv("AXG_KICK_VARIANT")) h->kick_variant = h->kick_variant_stack = atoi(e);
         if (const char* e = getenv("AXG_YPASS_VARIANT")) h->ypass_variant = atoi(e);
         // AXG_STRING_SPLIT: simplex iterations of the string fits' first kernel (same records)
         if (const char* e = getenv("AXG_STRING_SPLIT")) h->string_split = std::max(0, atoi(e));
@@ -851,7 +854,7 @@ static void stacked_step(axg_handle* h, const LatRef* lat, int nlat, int sidx, c
     const StepRef sr{nullptr, base, sidx};
     const KickScalars k{};
     if (!launch_kick_source_xfft<T, COMP>(h->stream, h->N, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                          nullptr, h->P, h->tw, k, p.dspa, 0.0, h->kick_variant, false, sr, lat, nlat))
+                                          nullptr, h->P, h->tw, k, p.dspa, 0.0, h->kick_variant_stack, false, sr, lat, nlat))
         throw Error(AXG_EINVAL, "stacked step: no fused pass for this size");
     launch_gw_ypass<T>(h->stream, h->N, h->P, nullptr, nullptr, h->L, h->plan, h->tw, h->ypass_variant, false, lat, nlat);
     GwStepScalars g;
@@ -996,7 +999,7 @@ extern "C" int axg_tune(axg_handle* h, int32_t reps, int32_t* variant, double* m
             }
         }
         AXG_HIP(hipStreamSynchronize(h->stream));
-        h->kick_variant = bestv;
+        h->kick_variant = h->kick_variant_stack = bestv;
         h->ypass_variant = ybestv;
         if (variant) *variant = bestv | (ybestv << 8);
     });
