@@ -652,15 +652,16 @@ __global__ void __launch_bounds__((p2_ztx<T, N>() * (N / 8))) gw_zpass_p2_kernel
 // LDS tile; then the threads share the tile's wavevectors (at most two each), whose accumulators
 // were loaded before the transforms.  Same arithmetic in the same order, so the accumulators are the
 // same bit for bit.  Kernel, us: 32^3 FP64 20.7 -> 7.6, FP32C 13.6 -> 7.6; 64^3 FP64 21.6 ->
-// 13.6, FP32C 17.6 -> 9.0; 96^3 FP64 36 -> 32.  Taken where the block fits 1024 threads and its
-// six tiles 80 KiB (two blocks a CU): FP64 to N = 96, FP32 to N = 64 (128^3 FP64, 96 KiB and one
-// block a CU, was slower, 56 -> 60 us), and where the grid's waves fit the chip at once: four
-// stacked 64^3 FP32C lattices (9216 waves) step in 66 us by themselves instead of 70, but beside
-// the other stacks of a mixed batch the larger blocks cost it 1 %.
+// 13.6, FP32C 17.6 -> 9.0.  Taken where the block fits 1024 threads and its six tiles 64 KiB (FP64 to N = 72,
+// FP32 to N = 64; with eight lattices stepped at once, one a thread, a step of 64^3 FP64 still falls from 21.7 to
+// 20.2 us).  Larger tiles leave a CU two blocks: 96^3 FP64 steps took 79.4 instead of 80.3 us alone, but 70 instead
+// of 60 with three lattices at once and 74 instead of 68 with eight; 128^3 FP64, one block a CU, was slower
+// alone.  And where the grid's waves fit the chip at once: four stacked 64^3 FP32C lattices (9216 waves) step
+// in 66 us by themselves instead of 70, but beside the other stacks of a mixed batch the larger blocks cost it 1 %.
 template <typename T, int N> constexpr int p2_zpar_threads() { return 6 * p2_ztx<T, N>() * (N / 8); }
 template <typename T, int N> constexpr bool p2_zpar()
 {
-    return !(sizeof(T) == 4 && P2<N>::R9) && p2_zpar_threads<T, N>() <= 1024 && 6 * N * p2_ztx<T, N>() * (int)sizeof(typename V2<T>::type) <= 80 * 1024;
+    return !(sizeof(T) == 4 && P2<N>::R9) && p2_zpar_threads<T, N>() <= 1024 && 6 * N * p2_ztx<T, N>() * (int)sizeof(typename V2<T>::type) <= 64 * 1024;
 }
 
 constexpr int64_t ZPAR_WAVES = 8192;  // 256 CUs x 4 SIMDs x 8 waves
